@@ -251,8 +251,8 @@ class AcousticPlan:
         return loss, g, tr
 
     def autotune(self, model: torch.Tensor, srcv: torch.Tensor, K: int, reps: int = 3):
-        """Pick the fastest (rows per wavefront, shots per workgroup) for the forward and adjoint
-        kernels on this plan (ads_acoustic_plan_autotune).  Returns the chosen shape."""
+        """Pick the fastest shape of the single-level forward and the adjoint's shots per workgroup
+        on this plan (ads_acoustic_plan_autotune).  Returns the chosen shape."""
         model = _dev(model, self.dtype)
         ws = self.workspace(K)
         out = (C.c_int * 6)()
@@ -271,18 +271,17 @@ class AcousticPlan:
         self.shape = tuple(shape)
 
     def set_blocking(self, levels: int = 2):
-        """Levels per interior-rectangle pass of the forward sweeps (2 = temporal blocking,
-        the default; bit-identical to 1)."""
+        """1: one launch per time level; 2 (the default): several levels per launch, bit-identical."""
         _lib.check(self.lib.ads_acoustic_plan_set_blocking(self.h, int(levels)))
 
     def set_frame_rows(self, rows: int = 0):
-        """Rows per item of the two-level PML-frame pass: 4, 8, 16, 32 or 64, or 0 to choose
-        per launch from the active shots and the launch's size (bit-identical results)."""
+        """Accepted for callers (0, 4, 8, 16, 32 or 64); changes nothing."""
         _lib.check(self.lib.ads_acoustic_plan_set_frame_rows(self.h, int(rows)))
 
     @property
     def blocking(self) -> int:
-        """Levels per pass in effect: 2 only when no source lies in the interior rectangle."""
+        """2 when several levels per launch are asked for and no source lies in the interior
+        rectangle, else 1 (ads_acoustic_plan_blocking)."""
         return int(self.lib.ads_acoustic_plan_blocking(self.h))
 
     def set_graph(self, enable: bool = True):

@@ -298,15 +298,14 @@ int ads_acoustic_plan_gradient(ads_acoustic_plan *plan, const void *model, const
                                void *traces, void *workspace, size_t ws_bytes, int64_t K,
                                ads_stream_t stream);
 
-/* Kernel-shape autotuner: times every candidate shape (rows per wavefront 1/2/4 x shots per
- * workgroup 1..32 x shots per batch 1/2, batch 2 only with 1-2 rows; the forward also 8 rows,
- * the streaming form of its two-level rectangle pass, one shot per wavefront) of the forward
- * and adjoint stencil kernels on this plan's own grid and shots for `reps` steps each, keeps
- * the fastest in the plan, and writes it to shape_out[6] = {fwd rows, fwd shots, fwd batch,
- * adj rows, adj shots, adj batch} (may be NULL).  Synchronises the stream; leaves the
- * workspace contents undefined.  ads_acoustic_plan_set_shape() sets a shape directly (same
- * 6-entry layout; forward rows 8 or 16 select the streaming rectangle where the two-level pass
- * applies and 2 rows elsewhere). */
+/* Kernel-shape autotuner: times the single-level forward's shapes (rows per wavefront 1/2/4 x shots per
+ * workgroup 1..32 x shots per batch 1/2, batch 2 only with 1-2 rows) and the adjoint's shots per workgroup
+ * (1..32) on this plan's own grid and shots for `reps` steps each, keeps the fastest in the plan, and
+ * writes them to shape_out[6] = {fwd rows, fwd shots, fwd batch, adj rows, adj shots, adj batch} (may be
+ * NULL).  Synchronises the stream; leaves the workspace contents undefined.
+ * ads_acoustic_plan_set_shape() sets a shape directly (same 6-entry layout).  The forward entries concern
+ * single-level stepping (ads_acoustic_plan_set_blocking(1); 8 or 16 rows stand for 2), the adjoint's shots
+ * per workgroup the multi-level adjoint; its rows and batch have no effect. */
 int ads_acoustic_plan_autotune(ads_acoustic_plan *plan, const void *model, const void *srcv,
                                void *workspace, size_t ws_bytes, int64_t K, int reps,
                                int *shape_out, ads_stream_t stream);
@@ -320,20 +319,15 @@ int ads_acoustic_plan_set_shape(ads_acoustic_plan *plan, const int *shape);
  * dropped by set_shape/autotune and at plan destruction. */
 int ads_acoustic_plan_set_graph(ads_acoustic_plan *plan, int enable);
 
-/* Temporal blocking of the forward sweeps (no counterpart in the reference): with levels = 2
- * (the default) the interior rectangle advances two time levels per pass (u^n and u^{n+1}
- * from u^{n-1}, u^{n-2}), which cuts its HBM traffic by a third; with PropagatorKernel 1 the
- * PML frame does too, in the same launch.  Results are bit-identical to levels = 1.  It
- * applies only when no source lies in the interior rectangle and to pairs of levels with the
- * same number of active shots; otherwise levels are stepped one at a time.
- * ads_acoustic_plan_blocking returns the levels per pass in effect (1 or 2). */
+/* Temporal blocking of the forward sweeps (no counterpart in the reference): with levels = 2 (the default)
+ * a launch advances several time levels (seven with PropagatorKernel 1 or 2, four with 0), each
+ * workgroup holding one tile of the grid with a halo in registers; with levels = 1 every level is a launch
+ * of its own.  Results are bit-identical.  ads_acoustic_plan_blocking returns 2 when levels = 2 is set and
+ * no source lies in the interior rectangle (the cells that no PML term reaches), else 1. */
 int ads_acoustic_plan_set_blocking(ads_acoustic_plan *plan, int levels);
 int ads_acoustic_plan_blocking(const ads_acoustic_plan *plan);
 
-/* Rows per item of the two-level PML-frame pass (no counterpart in the reference): 4, 8, 16,
- * 32 or 64 force that height; 0 (the default) chooses per launch the tallest height not above
- * the number of active shots whose per-wavefront walk over the item's rows, shot after shot,
- * stays well inside the launch's streaming time.  Results are bit-identical for every value. */
+/* Kept for callers: 0, 4, 8, 16, 32 or 64 are accepted and change nothing. */
 int ads_acoustic_plan_set_frame_rows(ads_acoustic_plan *plan, int rows);
 
 /* Plain drop-in of AcousticPropagatorSolver (Core.jl:562-620) on the plan's shots (every shot
@@ -421,13 +415,12 @@ int ads_elastic_forward_history(ads_elastic_plan *plan, const void *rho, const v
  * on its launch stream; ads_profile_end() waits for them and accumulates, per kernel class,
  * the summed duration, the launch count and the algorithmic HBM bytes of those launches
  * (compulsory per-cell traffic: acoustic forward w(4 + 4 f_pml), adjoint w(7 + 4 f_pml) for
- * PropagatorKernel 1; w(4 + 2 f_pml) and w(7 + 2 f_pml) for kernel 0 whose phi/psi updates
- * run in a separate pass; elastic forward w(8 + 4 f_x + 4 f_y) stress and w(5 + 4 f_x + 4 f_y)
+ * PropagatorKernel 1, w(4 + 2 f_pml) and w(7 + 2 f_pml) for kernel 0; elastic forward w(8 + 4 f_x + 4 f_y) stress and w(5 + 4 f_x + 4 f_y)
  * velocity phase, adjoint w(12 + 4 f_x + 4 f_y) per phase: the whole-step counts
  * w(13 + 8 f_x + 8 f_y) and w(24 + 8 f_x + 8 f_y) split by the fields each phase updates; the
  * fused elastic forward step, the default, is timed in ADS_PROF_EL_FWD_STRESS with the
- * whole-step count and leaves ADS_PROF_EL_FWD_VEL empty).  A launch that advances two time
- * levels (the acoustic forward's two-level pass) counts as two launches.
+ * whole-step count and leaves ADS_PROF_EL_FWD_VEL empty).  A launch that advances several time
+ * levels (the acoustic tiles) counts as that many launches.
  * ads_profile_begin_sampled(every) brackets only launches 0, every, 2*every, ... of each class
  * (counted from the begin call), so that a long timed run carries few events; the queried
  * duration, launch count and bytes then cover those launches alone.  ads_profile_begin() is
