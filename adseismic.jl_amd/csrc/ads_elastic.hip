@@ -1281,6 +1281,29 @@ __global__ __launch_bounds__(256) void el_adjs_rb(ElAdj<T> a, ElCoef<T> c, TileM
 // order (no atomics: the sums, like every other sum of the plan, are bitwise reproducible) and
 // added to the group's accumulators once per workgroup.  LDS: shots x terms x rows x WAVE.
 constexpr int SW_NW = 8, SW_CH_MAX = 32, SW_COLS = WAVE - 4, SW_LDS_ROWS = 64;  // shots x rows <= 64
+constexpr int STRM_CH = 8;  // the most rows a workgroup of the streaming adjoint takes unasked
+
+// Rows per wavefront of the streaming walks (forward and adjoint), `max` at most.  Taller chunks
+// re-read fewer halo rows but give fewer wavefronts, each walking its rows one after another at
+// 1 to 2 us a row: with few wavefronts that walk is the whole time of a launch.  The tallest
+// chunk that leaves 512 wavefronts per row of the chunk (4096 at 8 rows), and 12288 from 16 rows
+// on.  us per level, forward / adjoint velocity / adjoint stress phase:
+//   134 x 97, 4 shots, FP64:  8 rows 27.9 / 24.2 / 27.2 (136 wavefronts), 4: 20.8 / 16.9 / 19.0,
+//                             2: 15.7 / 13.2 / 15.1, 1: 15.9 / 12.6 / 14.2 (1088)
+//   300 x 250, 8 shots, FP64: 8 rows 35.9 / 35.7 / 38.3 (1520), 4: 28.7 / 34.1 / 37.7,
+//                             2: 35.5 / 35.8 / 39.9, 1: 44.8 / 44.5 / 51.3
+//   400 x 400, 8 shots, FP32: 8 rows 35.4 / 29.5 / 31.2 (3264), 4: 30.3 / 28.2 / 29.6,
+//                             2: 35.2 / 29.6 / 32.6, 1: 46.2 / 34.0 / 38.9
+//   600 x 600, 16 shots, FP32: forward 104 with 8 to 16 rows, 130 with 32 (3344)
+static int chunk_rows(int64_t nstrip, int64_t nrows, int64_t act, int max)
+{
+    int ch = 1;
+    for (int h = 2; h <= max; h *= 2) {
+        const int64_t waves = nstrip * (int64_t)cdiv(nrows, h) * act;
+        if (waves >= (h <= 8 ? int64_t(512) * h : int64_t(12288))) ch = h;
+    }
+    return ch;
+}
 
 struct StrmMap {
     int nstrip, nchunk, ngroup, nb, ch;
@@ -2555,8 +2578,9 @@ struct ElPlanBase {
     int rpt = 1, sg = 4;  // forward rectangle kernels: rows per wavefront, shots per workgroup
     // adjoint: shots per group (one wavefront each in the streaming rectangle kernels, whose
     // parameter terms are summed per group), streaming (1) or LDS-tiled (0) rectangle kernels,
-    // and the streaming kernels' rows per workgroup
-    int asg = NWAVES, strm = 2, strm_ch = 8;
+    // and the streaming kernels' rows per workgroup (0: chosen per launch, at most STRM_CH)
+    int asg = NWAVES, strm = 2, strm_ch = 0;
+    int strm_rows_max() const { return strm_ch > 0 ? std::min(strm_ch, SW_CH_MAX) : STRM_CH; }
     // forward: the fused streaming step (el_fwd_full) on the pitched layout, and its rows per
     // wavefront chunk (0: chosen per launch)
     int ffused = 1, fch = 0;
@@ -2607,7 +2631,7 @@ template <typename T> struct ElPlan : ElPlanBase {
     // must not change with the number of active shots (their LDS is sized for the plan's group).
     bool full_adjoint() const
     {
-        const size_t lds = (size_t)3 * asg * std::max(1, std::min(strm_ch, SW_CH_MAX)) * WAVE * sizeof(T);
+        const size_t lds = (size_t)3 * asg * strm_rows_max() * WAVE * sizeof(T);
         return strm == 2 && asg <= SW_NW && lds <= 65536 && (uint64_t)Npad * sizeof(T) < (uint64_t(1) << 32);
     }
     int64_t adj_groups() const { return (int64_t)cdiv(nshots, std::max(asg, 1)); }
@@ -2759,19 +2783,9 @@ template <typename T> struct ElPlan : ElPlanBase {
         const bool fuse = rr && li == 0 && nitems[li] > 0;  // rectangle + frame in one launch
         if (li == 0 && ffused && (uint64_t)Npad * sizeof(T) < (uint64_t(1) << 32)) {
             // one launch for both phases (the whole step's bytes, charged to the stress class)
-            // Taller chunks re-read fewer halo rows (8 rows: 1.19x the step's compulsory bytes,
-            // 32 rows: 1.0x at 600^2 x 16 shots) but give fewer wavefronts, each walking its
-            // rows one after another: below about 12 per SIMD the walk's latency is exposed
-            // (32 rows there: 130 against 104 us per level).  The tallest of 8, 16 and 32 rows
-            // that keeps that many wavefronts.
             StrmMap mp;
             mp.nstrip = (int)cdiv(NY + 2, FS_COLS);
-            mp.ch = fch;
-            if (mp.ch <= 0) {
-                mp.ch = 8;
-                for (int h = 16; h <= 32; h *= 2)
-                    if ((int64_t)mp.nstrip * cdiv(NX + 2, h) * act >= 12288) mp.ch = h;
-            }
+            mp.ch = fch > 0 ? fch : chunk_rows(mp.nstrip, NX + 2, act, 32);
             mp.nchunk = (int)cdiv(NX + 2, mp.ch);
             mp.ngroup = (int)cdiv(act, NWAVES);
             mp.nb = mp.nstrip * mp.nchunk * mp.ngroup;
@@ -2923,7 +2937,7 @@ template <typename T> struct ElPlan : ElPlanBase {
         const ElPar<T> par{w.par, w.par + Npad, w.par + 2 * Npad, w.par + 3 * Npad, w.par + 4 * Npad};
         // streaming kernels: their LDS (3 terms x shots x rows x WAVE values) must fit in 64 KiB,
         // else the LDS-tiled kernels run
-        const size_t strm_lds = (size_t)3 * a.Sg * std::max(1, std::min(strm_ch, SW_CH_MAX)) * WAVE * sizeof(T);
+        const size_t strm_lds = (size_t)3 * a.Sg * strm_rows_max() * WAVE * sizeof(T);
         // (the streaming kernels address one field of one shot with 32-bit byte offsets)
         const bool off32 = (uint64_t)Npad * sizeof(T) < (uint64_t(1) << 32);
         if (full_adjoint() && li == 0) {
@@ -2941,8 +2955,8 @@ template <typename T> struct ElPlan : ElPlanBase {
             }
             a.A = Ar;
             StrmMap sm;
-            sm.ch = std::max(1, std::min(strm_ch, SW_CH_MAX));
             sm.nstrip = (int)cdiv(NY + 2, SW_COLS);
+            sm.ch = strm_ch > 0 ? strm_rows_max() : chunk_rows(sm.nstrip, NX + 2, act, STRM_CH);
             sm.nchunk = (int)cdiv(NX + 2, sm.ch);
             sm.ngroup = ng;
             sm.nb = sm.nstrip * sm.nchunk * sm.ngroup;
@@ -2962,7 +2976,7 @@ template <typename T> struct ElPlan : ElPlanBase {
         }
         if (rr && strm && li == 0 && a.Sg <= SW_NW && strm_lds <= 65536 && off32) {
             StrmMap sm;
-            sm.ch = std::max(1, std::min(strm_ch, SW_CH_MAX));
+            sm.ch = strm_rows_max();
             sm.nstrip = (int)cdiv(a.R.jR - a.R.jL, SW_COLS);
             sm.nchunk = (int)cdiv(a.R.iR - a.R.iL, sm.ch);
             sm.ngroup = ng;

@@ -359,17 +359,17 @@ size_t ads_elastic_plan_workspace_size(const ads_elastic_plan *plan, int64_t K);
  * over the whole grid, x-direction stencils from registers, y-direction from neighbouring
  * lanes, the CPML memory cotangents formed on the fly), streaming over the interior rectangle
  * with separate frame passes (1) or LDS-tiled over the rectangle (0); rows per streaming
- * workgroup (1..32, default 8); shots per adjoint group (1..8, default 4; the parameter terms
- * are accumulated per group); rows x shots <= 64.  The streaming kernels need 3 x shots x rows
- * x 64 values of LDS; above 64 KiB (FP64 past 32 rows x shots) the LDS-tiled kernels run.
+ * workgroup (1..32; until set 1 to 8, chosen per launch from the number of wavefronts); shots
+ * per adjoint group (1..8, default 4; the parameter terms are accumulated per group); rows x
+ * shots <= 64.  The streaming kernels need 3 x shots x rows x 64 values of LDS; above 64 KiB (FP64 past 32 rows x shots) the LDS-tiled kernels run.
  * Changes the workspace layout (mode 2 keeps a second set of memory-variable cotangents):
  * call before ads_elastic_plan_workspace_size and the forward. */
 int ads_elastic_plan_set_adjoint_kernels(ads_elastic_plan *plan, int streaming, int rows,
                                          int shots);
 /* Forward kernels (no counterpart in the reference): fused = 1 (the default) steps a level in
  * one launch over the whole grid, the stress update two rows ahead of the velocity update in
- * registers, each wavefront walking `rows` rows of one shot (0, the default: 8, 16 or 32 rows,
- * the tallest that leaves enough wavefronts to fill the GPU); fused = 0 runs the
+ * registers, each wavefront walking `rows` rows of one shot (0, the default: 1 to 32 rows,
+ * the tallest chunk that leaves enough wavefronts to fill the GPU); fused = 0 runs the
  * stress and the velocity phase as two launches (interior rectangle tiles and the CPML frame
  * as streaming items).  Sources and receivers are applied after either. */
 int ads_elastic_plan_set_forward_kernels(ads_elastic_plan *plan, int fused, int rows);
