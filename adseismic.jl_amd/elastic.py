@@ -103,7 +103,8 @@ class ElasticPlan:
     def set_adjoint_kernels(self, streaming: int = 2, rows: int = 8, shots: int = 4) -> None:
         """Adjoint kernels (ads_elastic_plan_set_adjoint_kernels): 2 full-grid streaming, 1
         streaming rectangle with the frame passes, 0 LDS-tiled rectangle (True / False mean 1 /
-        X
+        0).  Until it is called the rows are chosen per launch.  It changes the workspace layout,
+        so call it before the forward."""
         _lib.check(self.lib.ads_elastic_plan_set_adjoint_kernels(self.h, int(streaming),
                                                                  int(rows), int(shots)))
         self._ws_K = None
