@@ -1295,10 +1295,13 @@ constexpr int STRM_CH = 8;  // the most rows a workgroup of the streaming adjoin
 //   400 x 400, 8 shots, FP32: 8 rows 35.4 / 29.5 / 31.2 (3264), 4: 30.3 / 28.2 / 29.6,
 //                             2: 35.2 / 29.6 / 32.6, 1: 46.2 / 34.0 / 38.9
 //   600 x 600, 16 shots, FP32: forward 104 with 8 to 16 rows, 130 with 32 (3344)
-static int chunk_rows(int64_t nstrip, int64_t nrows, int64_t act, int max)
+// min: the FP32 forward takes 8 rows at least.  The compiler contracts the first rows of a walk into
+// fused multiply-adds otherwise than the rest, so another height is another rounding, and the FP32
+// traces (and with them the misfit, by up to 5e-10 of it) would follow the number of active shots.
+static int chunk_rows(int64_t nstrip, int64_t nrows, int64_t act, int min, int max)
 {
-    int ch = 1;
-    for (int h = 2; h <= max; h *= 2) {
+    int ch = min;
+    for (int h = 2 * min; h <= max; h *= 2) {
         const int64_t waves = nstrip * (int64_t)cdiv(nrows, h) * act;
         if (waves >= (h <= 8 ? int64_t(512) * h : int64_t(12288))) ch = h;
     }
@@ -2785,7 +2788,7 @@ template <typename T> struct ElPlan : ElPlanBase {
             // one launch for both phases (the whole step's bytes, charged to the stress class)
             StrmMap mp;
             mp.nstrip = (int)cdiv(NY + 2, FS_COLS);
-            mp.ch = fch > 0 ? fch : chunk_rows(mp.nstrip, NX + 2, act, 32);
+            mp.ch = fch > 0 ? fch : chunk_rows(mp.nstrip, NX + 2, act, sizeof(T) == 4 ? 8 : 1, 32);
             mp.nchunk = (int)cdiv(NX + 2, mp.ch);
             mp.ngroup = (int)cdiv(act, NWAVES);
             mp.nb = mp.nstrip * mp.nchunk * mp.ngroup;
@@ -2956,7 +2959,7 @@ template <typename T> struct ElPlan : ElPlanBase {
             a.A = Ar;
             StrmMap sm;
             sm.nstrip = (int)cdiv(NY + 2, SW_COLS);
-            sm.ch = strm_ch > 0 ? strm_rows_max() : chunk_rows(sm.nstrip, NX + 2, act, STRM_CH);
+            sm.ch = strm_ch > 0 ? strm_rows_max() : chunk_rows(sm.nstrip, NX + 2, act, 1, STRM_CH);
             sm.nchunk = (int)cdiv(NX + 2, sm.ch);
             sm.ngroup = ng;
             sm.nb = sm.nstrip * sm.nchunk * sm.ngroup;

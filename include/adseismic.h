@@ -368,7 +368,7 @@ int ads_elastic_plan_set_adjoint_kernels(ads_elastic_plan *plan, int streaming, 
                                          int shots);
 /* Forward kernels (no counterpart in the reference): fused = 1 (the default) steps a level in
  * one launch over the whole grid, the stress update two rows ahead of the velocity update in
- * registers, each wavefront walking `rows` rows of one shot (0, the default: 1 to 32 rows,
+ * registers, each wavefront walking `rows` rows of one shot (0, the default: 1 to 32 rows, FP32 8 to 32,
  * the tallest chunk that leaves enough wavefronts to fill the GPU); fused = 0 runs the
  * stress and the velocity phase as two launches (interior rectangle tiles and the CPML frame
  * as streaming items).  Sources and receivers are applied after either. */
