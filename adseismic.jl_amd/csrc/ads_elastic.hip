@@ -23,6 +23,7 @@
 // (2 passes).  Sigma-type sources are removed from level n before its velocity VJP (fw3/fw4
 // read the stresses before injection).
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstring>
 #include <memory>
@@ -2548,7 +2549,24 @@ __global__ void el_model_in(const T *__restrict__ m, T *__restrict__ o, int NX, 
 }
 
 
+}  // namespace ads
+
+#include "ads_el_tile.h"
+
+namespace ads {
+
 // ------------------------------- plan ---------------------------------------------------
+// Levels per launch of the tile kernel.  A launch costs about 11 us on a small grid (tile table, states and
+// source lists one after another, the kernel's code fetched cold) and 5.6 us a level; each level also
+// takes 8 rows and columns off the 32 x 64 cells.  us per level with 1 / 2 / 3 levels, FP64:
+//   134 x 97, 4 shots 17.2 / 11.3 / 9.6;  200 x 200, 8 shots 26.4 / 19.1 / 27.3;
+//   300 x 250, 8 shots 30.1 / 27.5 / 42.0;  600 x 600, 8 shots 109 / 106 / 187
+constexpr int EL_TILE_LEVELS = 2;
+// Levels per launch, tile table and source lists.
+struct ElTilePlan {
+    int levels = 1, ntiles = 0;
+    DevBuf tiles, sptr, sgrp, skey;
+};
 struct ElPlanBase {
     virtual ~ElPlanBase() = default;
     ads_elastic_params p{};
@@ -2562,7 +2580,7 @@ struct ElPlanBase {
     DevBuf d_us_ptr, d_us_eptr, d_us_ent, d_nsrc, d_srcv_off, d_ur_ptr, d_ur_eptr, d_ur_ent;
     DevBuf d_rcv_ptr, d_trace_off, d_nstep;
     DevBuf d_us_key[2], d_ur_key[2], d_rcv_key[2];  // [0] pitched, [1] dense; key = cell*8+type
-    int64_t max_ur = 0;
+    int64_t max_ur = 0, max_rcv = 0;
     int64_t nkeys = 0;  // unique (cell, type) source keys over all shots
     // level slots and checkpoints keep the memory variables only outside this box, where some
     // CPML profile is non-zero (inside it they stay 0): nmv cells per shot and variable
@@ -2587,6 +2605,7 @@ struct ElPlanBase {
     // forward: the fused streaming step (el_fwd_full) on the pitched layout, and its rows per
     // wavefront chunk (0: chosen per launch)
     int ffused = 1, fch = 0;
+    ElTilePlan tile;  // register tiles of the forward
     // snapshot slots of the reversal schedule (< 0: one per segment start, the one-level scheme)
     int64_t snapshots = -1;
     int sub = 0;          // one MPIElastic subdomain (see ElCoef)
@@ -2620,6 +2639,7 @@ template <typename T> struct ElPlan : ElPlanBase {
         return c;
     }
     dim3 grid(int act) const { return dim3(cdiv(NY + 2, 64), cdiv(NX + 2, 4), act); }
+    static constexpr int TILE_R = 4;  // register rows per wavefront of the tiles
 
     struct WS {
         int64_t K, NS, M, S;  // interval, slots, segments, snapshot slots
@@ -2637,6 +2657,15 @@ template <typename T> struct ElPlan : ElPlanBase {
         const size_t lds = (size_t)3 * asg * strm_rows_max() * WAVE * sizeof(T);
         return strm == 2 && asg <= SW_NW && lds <= 65536 && (uint64_t)Npad * sizeof(T) < (uint64_t(1) << 32);
     }
+    // The tile kernels (32-bit byte offsets within one field of one shot) step forward unless the caller
+    // chose others: FP64 plans, and in either type the states that a dense history's cotangent is pulled back
+    // through (the history itself comes from the tiles).  FP32 traces come from el_fwd_full: the tiles
+    // contract its expressions otherwise, and the misfit would move (see chunk_rows).  us per level with the
+    // sources, el_fwd_full at its best rows / tiles:
+    //   134 x 97, 4 shots, FP64 20 / 11;  200 x 200, 8 shots 30 / 19;  300 x 250, 8 shots 33 / 27;
+    //   450 x 300, 2 shots 27 / 15;  600 x 600, 8 shots 118 / 106
+    bool off32() const { return (uint64_t)Npad * sizeof(T) < (uint64_t(1) << 32); }
+    bool tiled_forward(bool dense) const { return ffused && fch == 0 && off32() && (dense || sizeof(T) == 8); }
     int64_t adj_groups() const { return (int64_t)cdiv(nshots, std::max(asg, 1)); }
     void layout(WS &w, Carve &cv, int64_t K) const { layout(w, cv, K, snapshots); }
     void layout(WS &w, Carve &cv, int64_t K, int64_t snaps) const
@@ -2838,12 +2867,62 @@ template <typename T> struct ElPlan : ElPlanBase {
         return ADS_OK;
     }
 
-    int run_forward(const WS &w, int64_t lo, int64_t hi, const T *srcv, T *traces, int record,
+    // dense: the states behind a dense history's cotangent (see tiled_forward)
+    int run_forward(const WS &w, int64_t lo, int64_t hi, const T *srcv, T *traces, int record, bool dense,
                     hipStream_t st)
     {
+        if (tiled_forward(dense)) {
+            ElFwdTile<T> a{};
+            states(a, w);
+            a.rho = w.rho, a.lam = w.lam, a.mu = w.mu;
+            for (int64_t n = lo + 1; n <= hi; n += tile.levels)
+                ADS_TRY(forward_tiles(a, (int)n, (int)std::min<int64_t>(tile.levels, hi - n + 1), active[n], srcv,
+                                      (int)Pitch, st));
+            if (record && max_rcv > 0 && hi > lo) {
+                el_record<T><<<dim3(cdiv(max_rcv, 8), cdiv(hi - lo, 32), active[lo + 1]), 256, 0, st>>>(
+                    a.u, a.ls, a.fs, a.ss, a.NS, (int)lo, (int)hi, d_rcv_ptr.as<int64_t>(),
+                    d_rcv_key[0].template as<int64_t>(), d_nstep.as<int64_t>(), traces, d_trace_off.as<int64_t>());
+                ADS_LAUNCH_CHECK();
+            }
+            return ADS_OK;
+        }
         for (int64_t n = lo + 1; n <= hi; n++)
             ADS_TRY(step(slot(w, n - 1), slot(w, n), (int)n, active[n], w.rho, w.lam, w.mu, srcv,
                          traces, record, (int)Pitch, 0, st, pre_slot(w, n)));
+        return ADS_OK;
+    }
+    // the level slots as the tile kernels address them
+    void states(ElFwdTile<T> &a, const WS &w) const
+    {
+        a.u = w.seg;
+        a.ls = a.mls = level_elems();
+        a.fs = nshots * Npad, a.ss = Npad;
+        a.m = w.seg + 5 * nshots * Npad;
+        a.mfs = nshots * nmv, a.mss = nmv;
+        a.mb = mbox;
+        a.NS = (int)w.NS;
+        a.pre = w.pre, a.pls = std::max<int64_t>(nkeys, 1);
+    }
+    ElPoints points(const DevBuf &ptr, const DevBuf &grp, const DevBuf &key, const DevBuf &eptr, const DevBuf &ent) const
+    {
+        return ElPoints{ptr.as<int32_t>(), grp.as<int4>(), key.as<int2>(), eptr.as<int64_t>(), ent.as<int64_t>()};
+    }
+    int forward_tiles(ElFwdTile<T> &a, int n, int nt, int act, const T *srcv, int P, hipStream_t st)
+    {
+        if (act <= 0) return ADS_OK;
+        a.tiles = tile.tiles.as<int4>(), a.ntiles = tile.ntiles;
+        a.act = act, a.nb = tile.ntiles * act;
+        a.n = n, a.nt = nt;
+        a.c = coef(P);
+        a.nstep = d_nstep.as<int64_t>();
+        a.src = points(tile.sptr, tile.sgrp, tile.skey, d_us_eptr, d_us_ent);
+        a.srcv = srcv, a.srcv_off = d_srcv_off.as<int64_t>(), a.nsrc = d_nsrc.as<int64_t>();
+        const unsigned nb = (unsigned)(cdiv(a.nb, NXCD) * NXCD);
+        const int pr = prof_start(ADS_PROF_EL_FWD_STRESS, st);
+        if (sub) el_fwd_tile<T, 1, TILE_R><<<nb, WAVE * ET_NW, 0, st>>>(a);
+        else el_fwd_tile<T, 0, TILE_R><<<nb, WAVE * ET_NW, 0, st>>>(a);
+        prof_stop(pr, st, (double)act * PX * PY * nt * sizeof(T) * (13.0 + 8.0 * f_x + 8.0 * f_y), nt);
+        ADS_LAUNCH_CHECK();
         return ADS_OK;
     }
 
@@ -2860,7 +2939,7 @@ template <typename T> struct ElPlan : ElPlanBase {
     }
 
     int forward(const void *rho, const void *lam, const void *mu, const void *srcv, void *traces,
-                void *ws, size_t wsb, int64_t K, hipStream_t st)
+                void *ws, size_t wsb, int64_t K, hipStream_t st, bool dense = false)
     {
         WS w;
         ADS_TRY(check_ws(w, ws, wsb, K));
@@ -2878,7 +2957,7 @@ template <typename T> struct ElPlan : ElPlanBase {
             int64_t a = m * w.K, b = std::min<int64_t>(a + w.K, NMAX);
             if (pi < path.size() && path[pi].first == m)
                 ADS_TRY(copy_state(ckpt(w, path[pi++].second), slot(w, a), active[std::min<int64_t>(a + 1, NMAX)], st));
-            ADS_TRY(run_forward(w, a, b, (const T *)srcv, (T *)traces, traces != nullptr, st));
+            ADS_TRY(run_forward(w, a, b, (const T *)srcv, (T *)traces, traces != nullptr, dense, st));
         }
         return ADS_OK;
     }
@@ -3080,7 +3159,7 @@ template <typename T> struct ElPlan : ElPlanBase {
             {
                 for (int64_t m = m0; m < m1; m++) {
                     const int64_t a = m * w.K, b = std::min<int64_t>(a + w.K, pl->NMAX);
-                    ADS_TRY(pl->run_forward(w, a, b, sv, nullptr, 0, st));
+                    ADS_TRY(pl->run_forward(w, a, b, sv, nullptr, 0, dense_hist != nullptr, st));
                 }
                 return ADS_OK;
             }
@@ -3126,9 +3205,24 @@ template <typename T> struct ElPlan : ElPlanBase {
                         void *hist, void *scratch, hipStream_t st)
     {
         const int64_t L = NMAX + 1, N = Ndense;
-        ADS_HIP(hipMemsetAsync(hist, 0, (size_t)nshots * 5 * L * N * sizeof(T), st));
         T *mem = (T *)scratch;
         ADS_HIP(hipMemsetAsync(mem, 0, (size_t)2 * 8 * nshots * N * sizeof(T), st));
+        if ((uint64_t)N * sizeof(T) < (uint64_t(1) << 32)) {
+            // level 0 is zero; the tiles write every cell of the others
+            ADS_HIP(hipMemset2DAsync(hist, (size_t)L * N * sizeof(T), 0, (size_t)N * sizeof(T), (size_t)nshots * 5, st));
+            ElFwdTile<T> t{};
+            t.u = (T *)hist, t.ls = N, t.fs = L * N, t.ss = 5 * L * N, t.NS = INT_MAX;
+            t.mfs = (int64_t)nshots * N, t.mss = N;
+            t.rho = (const T *)rho, t.lam = (const T *)lam, t.mu = (const T *)mu;
+            T *cur = mem, *nxt = mem + (size_t)8 * nshots * N;
+            for (int64_t n = 1; n <= NMAX; n += tile.levels, std::swap(cur, nxt)) {
+                t.m = cur, t.mo = nxt;
+                ADS_TRY(forward_tiles(t, (int)n, (int)std::min<int64_t>(tile.levels, NMAX - n + 1), (int)nshots,
+                                      (const T *)srcv, (int)(NY + 2), st));
+            }
+            return ADS_OK;
+        }
+        ADS_HIP(hipMemsetAsync(hist, 0, (size_t)nshots * 5 * L * N * sizeof(T), st));
         auto lvl = [&](int64_t n) {
             El<T> e;
             for (int q = 0; q < 5; q++) {
@@ -3351,6 +3445,27 @@ static int build_el_plan(const ads_elastic_params *p, const ads_shot_geometry *g
             if (!items.empty()) ADS_TRY(P->d_ring[li].upload(items));
         }
     }
+    {
+        ElTilePlan &t = P->tile;
+        constexpr int R = ElPlan<T>::TILE_R;
+        t.levels = EL_TILE_LEVELS;
+        const std::vector<ElTileHost> h = el_tiles((int)P->NX, (int)P->NY, t.levels, R * ET_NW, P->rect[1]);
+        t.ntiles = (int)h.size();
+        std::vector<int4> tab;
+        for (const ElTileHost &x : h) {
+            tab.push_back(make_int4(x.i0, x.i1, x.j0, x.j1));
+            tab.push_back(make_int4(x.ie, x.je, x.ne | x.ce << 16, x.kind));
+        }
+        ADS_TRY(t.tiles.upload(tab));
+        std::vector<int64_t> key(si.size());
+        for (size_t e = 0; e < si.size(); e++) key[e] = (si[e] * P->Pitch + sj[e]) * 8 + st_[e];
+        const CellLists us = build_cell_lists(ns, sp.data(), key);
+        const ElPointLists l = el_point_lists(h, R, P->Pitch, us.shot_ptr, us.cell);
+        ADS_TRY(t.sptr.upload(l.ptr));
+        ADS_TRY(t.sgrp.upload(l.grp));
+        ADS_TRY(t.skey.upload(l.key));
+        for (int64_t q = 0; q < ns; q++) P->max_rcv = std::max(P->max_rcv, rp[q + 1] - rp[q]);
+    }
     ADS_TRY(P->d_nsrc.upload(nsrc));
     ADS_TRY(P->d_srcv_off.upload(soff));
     ADS_TRY(P->d_rcv_ptr.upload(rp));
@@ -3548,7 +3663,7 @@ int ads_elastic_plan_backward_dense(ads_elastic_plan *plan, const void *rho, con
         ADS_FAIL(ADS_ERR_ARG, "null argument");
     return el_dispatch(plan, [&](auto &P) -> int {
         if (P.NMAX != P.p.NSTEP) ADS_FAIL(ADS_ERR_SHAPE, "dense cotangents need nstep == NSTEP for every shot");
-        ADS_TRY(P.forward(rho, lam, mu, srcv, nullptr, ws, wsb, K, S(stream)));
+        ADS_TRY(P.forward(rho, lam, mu, srcv, nullptr, ws, wsb, K, S(stream), true));
         return P.backward(srcv, nullptr, grad_hist, grad_rho, grad_lam, grad_mu, ws, wsb, K, S(stream));
     });
 }

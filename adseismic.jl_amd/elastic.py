@@ -111,7 +111,8 @@ class ElasticPlan:
 
     def set_forward_kernels(self, fused: int = 1, rows: int = 0) -> None:
         """Forward kernels (ads_elastic_plan_set_forward_kernels): 1 one fused launch per level
-        walking `rows` rows per wavefront (0: chosen from the grid and the active shots), 0 the
+        walking `rows` rows per wavefront (0: FP32 chosen from the grid and the active shots, FP64
+        two levels per launch over register tiles), 0 the
         stress and velocity phases as two launches."""
         _lib.check(self.lib.ads_elastic_plan_set_forward_kernels(self.h, int(fused), int(rows)))
 

@@ -368,10 +368,12 @@ int ads_elastic_plan_set_adjoint_kernels(ads_elastic_plan *plan, int streaming, 
                                          int shots);
 /* Forward kernels (no counterpart in the reference): fused = 1 (the default) steps a level in
  * one launch over the whole grid, the stress update two rows ahead of the velocity update in
- * registers, each wavefront walking `rows` rows of one shot (0, the default: 1 to 32 rows, FP32 8 to 32,
- * the tallest chunk that leaves enough wavefronts to fill the GPU); fused = 0 runs the
+ * registers, each wavefront walking `rows` rows of one shot (0, the default: FP32 8 to 32 rows,
+ * the tallest chunk that leaves enough wavefronts to fill the GPU; FP64 plans step two levels per
+ * launch over register tiles instead); fused = 0 runs the
  * stress and the velocity phase as two launches (interior rectangle tiles and the CPML frame
- * as streaming items).  Sources and receivers are applied after either. */
+ * as streaming items).  Sources and receivers are applied after either (in the tiles: within).
+ * Dense histories always come from the tiles, where one field of one shot is below 4 GiB. */
 int ads_elastic_plan_set_forward_kernels(ads_elastic_plan *plan, int fused, int rows);
 /* As ads_acoustic_plan_choose_interval, over the NSTEP elastic levels. */
 int64_t ads_elastic_plan_choose_interval(const ads_elastic_plan *plan, size_t budget_bytes);
