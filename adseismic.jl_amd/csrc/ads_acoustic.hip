@@ -399,13 +399,7 @@ struct AcPlanBase {
     int ntiles = 0;
     DevBuf d_tiles, d_ts_ptr, d_ts_cell, d_ts_ent, d_tr_ptr, d_tr_cell, d_tr_ent;
     DevBuf d_nstep32;
-    // Levels per launch of the tile kernels.  More levels read and write the state less often, but widen
-    // the halo; kernel 0's PML loses two halo cells per level.  us per level, forward + adjoint, for
-    // 4 / 5 / 6 / 7 / 8 / 10 levels with kernel 1: 1000^2 x 32 shots FP32 65 + 95, 58 + 85, 61 + 89, 54 + 86,
-    // 60 + 88, 61 + 102; 2000^2 x 64 388 + 525, 388 + 494, 383 + 496, 362 + 457, 382 + 472, 385 + 531; for
-    // 2 / 3 / 4 / 5 with kernel 0: 400 x 800 x 24 FP32 22 + 48, 19 + 40, 20 + 42, 21 + 48; 200 x 66 x 8 FP64
-    // 5.7 + 8.3, 4.4 + 6.3, 3.7 + 5.5, 4.6 + 7.6.
-    int tile_levels = 4;
+    int tile_levels = 4;  // levels per launch of the tile kernels (choose_levels)
     // hipGraph replay of whole checkpoint segments (forward sweep, recomputation, adjoint
     // sweep), keyed by everything the captured launches depend on
     struct GraphKey {
@@ -1095,6 +1089,34 @@ template <typename T> struct AcPlan : AcPlanBase {
 };
 
 // The tiles of the multi-level kernels and their point lists.
+// Levels per launch.  More levels read and write the state and launch less often, but widen the halo (by
+// one cell a level, kernel 0's PML by two) and so need more tiles.
+// Where all workgroups of an adjoint launch are on the card at once (one per CU in FP64, two in FP32) a
+// launch takes as long as one of them, and the more levels the better: the most that still fit.  ms of a
+// call with kernel 0 for 4 / 5 / 6 / 7 levels (largest that fits in brackets): 200^2 solver FP64 9.8 / 9.0 /
+// 8.3 / [7.9]; 300 x 280 solver FP64 4.8 / 4.7 / [4.4] / 5.6; 1501 x 401 forward FP32 3.25 / [2.9] / 3.4 /
+// 4.6; 200 x 66, 8 shots, FP64 [15.6] / 21.0 / 19.4 / 30.9; 300 x 200, 1 shot, FP32 2.4 / 2.2 / 2.0 / [1.9].
+// Beyond that the work counts: the tiles, a PML tile at 2.2 of a plain one (half the rows, four times the
+// instructions), per level.  ms for 3 / 4 levels, the model's choice in brackets: 400 x 800, 24 shots, FP32
+// [31.7] / 33.9; 1000^2, 32 shots, FP32 24.2 / [22.4]; 700 x 600, 16 shots, FP64 10.4 / [10.0].  Kernel 1
+// takes 7: us per level, forward + adjoint, for 5 / 6 / 7 / 8 / 10 levels at 1000^2 x 32 shots FP32 66 + 99, 65 +
+// 101, 63 + 101, 63 + 103, 71 + 123; at 2000^2 x 64 396 + 538, 388 + 498, 380 + 499, 401 + 505, 421 + 576.
+static int choose_levels(int variant, int64_t nshots, size_t elem, const Rect &R, const TileGrid &g)
+{
+    const int64_t fit = elem == 4 ? 512 : 256;
+    for (int L = variant == 0 ? 7 : 12; L >= (variant == 0 ? 3 : 8); L--)
+        if ((int64_t)make_tiles(variant, L, R, g).size() * nshots <= fit) return L;
+    if (variant == 1) return 7;
+    int best = 4;
+    double least = 0.0;
+    for (int L = 3; L <= 5; L++) {
+        double c = 0.0;
+        for (const TileHost &t : make_tiles(variant, L, R, g)) c += t.kind == TILE_PLAIN ? 1.0 : 2.2;
+        if (least == 0.0 || c / L < least) least = c / L, best = L;
+    }
+    return best;
+}
+
 template <typename T>
 static int build_tiles(AcPlan<T> *P, const Rect &R, const std::vector<int64_t> &sp,
                        const std::vector<int64_t> &si, const std::vector<int64_t> &sj, const std::vector<int64_t> &rp,
@@ -1102,8 +1124,9 @@ static int build_tiles(AcPlan<T> *P, const Rect &R, const std::vector<int64_t> &
 {
     const int NX = (int)P->NX, NY = (int)P->NY;
     const std::vector<T> sx(P->sx.begin(), P->sx.end()), ty(P->ty.begin(), P->ty.end());
-    const std::vector<TileHost> tiles =
-        make_tiles(P->variant, P->tile_levels, R, tile_grid(sx, ty, TILE_WAVES * TILE_RN, TILE_WAVES * TILE_RP, 1));
+    const TileGrid grid = tile_grid(sx, ty, TILE_WAVES * TILE_RN, TILE_WAVES * TILE_RP, 1);
+    P->tile_levels = choose_levels(P->variant, P->nshots, sizeof(T), R, grid);
+    const std::vector<TileHost> tiles = make_tiles(P->variant, P->tile_levels, R, grid);
     std::vector<int4> t;
     for (const TileHost &q : tiles) {
         t.push_back(make_int4(q.i0, q.i1, q.j0, q.j1));
@@ -1273,7 +1296,6 @@ static int build_plan(const ads_acoustic_params *p, const ads_shot_geometry *g, 
     ADS_TRY(P->d_trace_off.upload(toff));
     ADS_TRY(P->d_nstep_sorted.upload(P->nstep_sorted));
     ADS_TRY(P->d_nstep32.upload(std::vector<int32_t>(P->nstep_sorted.begin(), P->nstep_sorted.end())));
-    P->tile_levels = P->variant == 1 ? 7 : 4;
     ADS_TRY(build_tiles(P, plain, sp, si, sj, rp, ri, rj));
     // Shots per adjoint workgroup: a workgroup keeps its model rows and dL/dC in registers over its shots,
     // so more shots save their traffic as long as every CU still has four workgroups (1000^2 x 32 shots
