@@ -484,11 +484,11 @@ __device__ inline void fwd_tile_body(const FwdTile<T> &a, const TileView &t, int
     }
 }
 
-// RN (RP): rows per wavefront of a plain (PML) tile; VEC columns per lane.  What bounds it: with 7 levels
-// per launch at 1000^2 x 32 shots FP32 (54 us per level; one level per launch took 104) about 3.9 TB/s move,
-// and the vector units issue half of the time; the two do not overlap fully between a workgroup's load
-// and compute phases, so three workgroups per CU (80 VGPRs, a few spilled) are asked for: 66 against 68 us
-// with the 2.5 that the compiler chooses, 77 with four (64 VGPRs).
+// RN (RP): rows per wavefront of a plain (PML) tile; VEC columns per lane.  What bounds it: at 1000^2 x 32
+// shots FP32 with 7 levels per launch (63 us per level; one level per launch takes 104) the vector units
+// issue two thirds of the time, half of that for the PML tiles and 40 % for the halo, and 3.3 TB/s move,
+// mostly stores; a workgroup's loads do not overlap its own levels, so several per CU have to.
+// FP32 asks for three (80 VGPRs, a few spilled): 63 us, two 63, four (64 VGPRs) 74.
 template <typename T, int V, int RN, int RP, int VEC, int NW>
 __global__ __launch_bounds__(NW *WAVE) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 6 : 4)))
 void ac_fwd_tile(const FwdTile<T> a)
@@ -804,9 +804,9 @@ __device__ inline void adj_tile_body(const AdjTile<T> &a, const TileView &t, int
     }
 }
 
-// Bounds as in the forward; 1000^2 x 32 shots FP32, 7 levels per launch: 86 us per level (one level per
-// launch and a receiver launch: 178).  Two workgroups per CU in FP32 (128 VGPRs with a few spilled): 87
-// against 123 us with one (no spills).
+// Bounds as in the forward; 1000^2 x 32 shots FP32, 7 levels per launch: 94 us per level (one level per
+// launch and a receiver launch: 178).  Two workgroups per CU in FP32 (128 VGPRs with a few spilled): 100
+// against 147 us with one (no spills) and 203 with three, eight shots per workgroup.
 template <typename T, int V, int RN, int RP, int VEC, int NW, bool DENSE>
 __global__ __launch_bounds__(NW *WAVE) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 4 : 2)))
 void ac_adj_tile(const AdjTile<T> a)

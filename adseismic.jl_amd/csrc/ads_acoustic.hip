@@ -354,9 +354,10 @@ struct Shape {
 };
 
 // Shape of the tile kernels: 8 wavefronts of 8 rows (plain tiles) or 4 rows (PML tiles, whose state is
-// larger) by 64 columns.  16 wavefronts, 2, 4 or 16 rows of a plain tile, 8 rows of a PML tile and two
-// columns per lane were all slower (1000^2 x 32 shots FP32, forward: 66 us per level; 8 / 8 rows 77, 4 / 4
-// rows 82, 16 / 4 rows 69, two columns 67, and the adjoint 267 instead of 88 with two columns).
+// larger) by 64 columns.  Compared at 1000^2 x 32 shots FP32, each against the 8 / 4 of its time: forward us per
+// level with 16 wavefronts of 4 / 4 rows 69 against 66, 8 / 8 rows 77, 4 / 4 rows 82, two columns per lane 67 (the
+// adjoint 267 against 88).  5 and 6 rows of a PML tile: the whole gradient 84.6 and 99.0 ms against 82.5,
+// and 200 x 66 x 8 shots FP64 18.0 and 26.7 against 15.6.
 constexpr int TILE_WAVES = 8, TILE_RN = 8, TILE_RP = 4;
 
 struct AcPlanBase {
@@ -1298,9 +1299,10 @@ static int build_plan(const ads_acoustic_params *p, const ads_shot_geometry *g, 
     ADS_TRY(P->d_nstep32.upload(std::vector<int32_t>(P->nstep_sorted.begin(), P->nstep_sorted.end())));
     ADS_TRY(build_tiles(P, plain, sp, si, sj, rp, ri, rj));
     // Shots per adjoint workgroup: a workgroup keeps its model rows and dL/dC in registers over its shots,
-    // so more shots save their traffic as long as every CU still has four workgroups (1000^2 x 32 shots
-    // FP32, 4 levels per launch: 132, 97 and 90 us per level for 1, 4 and 8 shots; 200 x 66 x 8: 5.5, 15, 27).
-    P->adj_shape.sg = (int)std::min<int64_t>(8, std::max<int64_t>(1, (int64_t)P->ntiles * ns / 1024));
+    // so more shots save their traffic as long as every CU still has four workgroups; past four shots the
+    // last workgroups' tail costs more.  us per level, FP32, for 1 / 2 / 4 / 8 shots: 1000^2 x 32 shots 119 /
+    // 98 / 94 / 100, kernel 0 - / 152 / 137 / 147; for 2 / 4 / 8: 2000^2 x 64 546 / 490 / 499.
+    P->adj_shape.sg = (int)std::min<int64_t>(4, std::max<int64_t>(1, (int64_t)P->ntiles * ns / 1024));
     return ADS_OK;
 }
 

@@ -57,10 +57,10 @@ TRAFFIC_FILES = {
 }
 
 
-# Kernel shape of the acoustic plan on the benchmark workloads: the adjoint's shots per workgroup (8) is
+# Kernel shape of the acoustic plan on the benchmark workloads: the adjoint's shots per workgroup (4) is
 # what the multi-level tile kernels take from it, and is the plan's own choice at both sizes; the
 # other entries concern single-level stepping.
-DEFAULT_SHAPE = "2,16,1,2,8,1"
+DEFAULT_SHAPE = "2,16,1,2,4,1"
 
 
 def measured_traffic(kernel, shape, path):
