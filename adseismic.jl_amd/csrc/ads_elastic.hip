@@ -2528,13 +2528,22 @@ __global__ __launch_bounds__(256) void el_adj_start(
     A.f((int)(key & 7), s)[key >> 3] += R;
 }
 
-// dense cotangent of the 5 field histories at level n (full-history pullback)
+// Start of an adjoint level of the full-history pullback, one launch: the dense cotangent of the 5 field
+// histories at level n, and in the last row of blocks the pre-injection stresses of the level's state
+// (as in el_adj_start).  The two touch different arrays.
 template <typename T>
-__global__ void el_adj_dense(El<T> A, ElC<T> D, int NX, int NY, int P)
+__global__ __launch_bounds__(256) void el_adj_dense(El<T> A, ElC<T> D, int NX, int NY, int P, El<T> Sn, int n, SrcTab st,
+                                                    const T *__restrict__ srcv, T *__restrict__ pre)
 {
+    const int s = blockIdx.z;
+    if (blockIdx.y + 1 == gridDim.y) {
+        if (blockIdx.x == 0)
+            el_src_rcv_body(Sn, n, st.us_ptr, st.us_key, st.us_eptr, st.us_ent, srcv, st.srcv_off, st.nsrc, st.rcv_ptr,
+                            st.rcv_key, st.nstep, (T *)nullptr, st.trace_off, 2, pre, s);
+        return;
+    }
     const int j = blockIdx.x * 64 + (threadIdx.x & 63);
     const int i = blockIdx.y * 4 + (threadIdx.x >> 6);
-    const int s = blockIdx.z;
     if (j >= NY + 2 || i >= NX + 2) return;
     const int64_t ij = (int64_t)i * P + j, d = (int64_t)i * (NY + 2) + j;  // D is dense
     for (int q = 0; q < 5; q++) A.f(q, s)[ij] += D.f(q, s)[d];
@@ -2976,12 +2985,17 @@ template <typename T> struct ElPlan : ElPlanBase {
                              d_srcv_off.as<int64_t>(),  d_nsrc.as<int64_t>(),
                              d_rcv_ptr.as<int64_t>(),   d_rcv_key[li].template as<int64_t>(),
                              d_nstep.as<int64_t>(),     d_trace_off.as<int64_t>()};
-            el_adj_start<T><<<dim3(nxi + 1, act), 256, 0, st>>>(
-                A, Sn, n, d_ur_ptr.as<int64_t>(), d_ur_key[li].template as<int64_t>(), d_ur_eptr.as<int64_t>(),
-                d_ur_ent.as<int64_t>(), d_nstep.as<int64_t>(), resid, d_trace_off.as<int64_t>(), nxi, tab, srcv,
-                pre_slot(w, n));
+            if (dense) {  // no trace residual beside a dense cotangent
+                dim3 g = grid(act);
+                g.y++;
+                el_adj_dense<T><<<g, 256, 0, st>>>(A, *dense, (int)NX, (int)NY, P, Sn, n, tab, srcv, pre_slot(w, n));
+            } else {
+                el_adj_start<T><<<dim3(nxi + 1, act), 256, 0, st>>>(
+                    A, Sn, n, d_ur_ptr.as<int64_t>(), d_ur_key[li].template as<int64_t>(), d_ur_eptr.as<int64_t>(),
+                    d_ur_ent.as<int64_t>(), d_nstep.as<int64_t>(), resid, d_trace_off.as<int64_t>(), nxi, tab, srcv,
+                    pre_slot(w, n));
+            }
         }
-        if (dense) el_adj_dense<T><<<grid(act), 256, 0, st>>>(A, *dense, (int)NX, (int)NY, P);
         ElAdj<T> a;
         a.A = A;
         a.Sn = cst(Sn);
