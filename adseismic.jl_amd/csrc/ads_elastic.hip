@@ -1284,28 +1284,33 @@ __global__ __launch_bounds__(256) void el_adjs_rb(ElAdj<T> a, ElCoef<T> c, TileM
 constexpr int SW_NW = 8, SW_CH_MAX = 32, SW_COLS = WAVE - 4, SW_LDS_ROWS = 64;  // shots x rows <= 64
 constexpr int STRM_CH = 8;  // the most rows a workgroup of the streaming adjoint takes unasked
 
-// Rows per wavefront of the streaming walks (forward and adjoint), `max` at most.  Taller chunks
-// re-read fewer halo rows but give fewer wavefronts, each walking its rows one after another at
-// 1 to 2 us a row: with few wavefronts that walk is the whole time of a launch.  The tallest
-// chunk that leaves 512 wavefronts per row of the chunk (4096 at 8 rows), and 12288 from 16 rows
-// on.  us per level, forward / adjoint velocity / adjoint stress phase:
-//   134 x 97, 4 shots, FP64:  8 rows 27.9 / 24.2 / 27.2 (136 wavefronts), 4: 20.8 / 16.9 / 19.0,
-//                             2: 15.7 / 13.2 / 15.1, 1: 15.9 / 12.6 / 14.2 (1088)
-//   300 x 250, 8 shots, FP64: 8 rows 35.9 / 35.7 / 38.3 (1520), 4: 28.7 / 34.1 / 37.7,
-//                             2: 35.5 / 35.8 / 39.9, 1: 44.8 / 44.5 / 51.3
-//   400 x 400, 8 shots, FP32: 8 rows 35.4 / 29.5 / 31.2 (3264), 4: 30.3 / 28.2 / 29.6,
-//                             2: 35.2 / 29.6 / 32.6, 1: 46.2 / 34.0 / 38.9
-//   600 x 600, 16 shots, FP32: forward 104 with 8 to 16 rows, 130 with 32 (3344)
-// min: the FP32 forward takes 8 rows at least.  The compiler contracts the first rows of a walk into
-// fused multiply-adds otherwise than the rest, so another height is another rounding, and the FP32
-// traces (and with them the misfit, by up to 5e-10 of it) would follow the number of active shots.
-static int chunk_rows(int64_t nstrip, int64_t nrows, int64_t act, int min, int max)
+// Rows per wavefront of the streaming walks.  Taller chunks re-read fewer halo rows but give fewer
+// wavefronts, each walking its rows one after another at 1 to 2 us a row.
+// Adjoint: where all wavefronts are on the card at once (4 per SIMD in FP32, 2 in FP64, by their
+// registers) a launch takes as long as one walk: the fewest rows for which they are, else 8.  us per level,
+// velocity / stress phase, for 8 / 4 / 2 / 1 rows, the rule's choice in brackets:
+//   134 x 97, 4 shots, FP64   24.2 / 27.2   16.9 / 19.0   13.2 / 15.1  [12.6 / 14.2]
+//   200 x 200, 8 shots, FP64  26.5 / 29.0  [22.7 / 24.3]  26.1 / 29.0   30.8 / 35.2
+//   661 x 144, 6 shots, FP64 [37.5 / 40.8]  40.1 / 44.3   48.0 / 54.3   63.5 / 73.2
+//   250 x 200, 4 shots, FP32  19.7 / 22.6   13.7 / 16.5   11.9 / 14.1  [11.9 / 13.8]
+//   600 x 200, 3 shots, FP32  23.1 / 26.3   18.0 / 20.6  [14.4 / 16.9]  18.4 / 21.4
+//   250 x 200, 12 shots, FP32 24.5 / 27.2  [18.7 / 21.1]  21.1 / 24.9   25.2 / 30.1
+//   490 x 235, 9 shots, FP32 [29.3 / 32.5]  30.2 / 35.2   32.7 / 38.1   41.8 / 51.0
+// Forward (FP32 plans; FP64 takes the tiles): the tallest of 8, 16 and 32 rows that leaves 12288
+// wavefronts (600 x 600, 16 shots: 104 us with 8 to 16 rows, 130 with 32).  Not below 8: the compiler
+// contracts the first rows of a walk into fused multiply-adds otherwise than the rest, so another height is
+// another rounding, and the FP32 traces (and with them the misfit, by up to 5e-10 of it) would move.
+static int adjoint_rows(int64_t nstrip, int64_t nrows, int64_t act, size_t elem)
 {
-    int ch = min;
-    for (int h = 2 * min; h <= max; h *= 2) {
-        const int64_t waves = nstrip * (int64_t)cdiv(nrows, h) * act;
-        if (waves >= (h <= 8 ? int64_t(512) * h : int64_t(12288))) ch = h;
-    }
+    for (int h = 1; h < STRM_CH; h *= 2)
+        if (nstrip * (int64_t)cdiv(nrows, h) * act <= (elem == 4 ? 4096 : 2048)) return h;
+    return STRM_CH;
+}
+static int forward_rows(int64_t nstrip, int64_t nrows, int64_t act)
+{
+    int ch = 8;
+    for (int h = 16; h <= 32; h *= 2)
+        if (nstrip * (int64_t)cdiv(nrows, h) * act >= 12288) ch = h;
     return ch;
 }
 
@@ -2669,7 +2674,7 @@ template <typename T> struct ElPlan : ElPlanBase {
     // The tile kernels (32-bit byte offsets within one field of one shot) step forward unless the caller
     // chose others: FP64 plans, and in either type the states that a dense history's cotangent is pulled back
     // through (the history itself comes from the tiles).  FP32 traces come from el_fwd_full: the tiles
-    // contract its expressions otherwise, and the misfit would move (see chunk_rows).  us per level with the
+    // contract its expressions otherwise, and the misfit would move (see forward_rows).  us per level with the
     // sources, el_fwd_full at its best rows / tiles:
     //   134 x 97, 4 shots, FP64 20 / 11;  200 x 200, 8 shots 30 / 19;  300 x 250, 8 shots 33 / 27;
     //   450 x 300, 2 shots 27 / 15;  600 x 600, 8 shots 118 / 106
@@ -2826,7 +2831,7 @@ template <typename T> struct ElPlan : ElPlanBase {
             // one launch for both phases (the whole step's bytes, charged to the stress class)
             StrmMap mp;
             mp.nstrip = (int)cdiv(NY + 2, FS_COLS);
-            mp.ch = fch > 0 ? fch : chunk_rows(mp.nstrip, NX + 2, act, sizeof(T) == 4 ? 8 : 1, 32);
+            mp.ch = fch > 0 ? fch : forward_rows(mp.nstrip, NX + 2, act);
             mp.nchunk = (int)cdiv(NX + 2, mp.ch);
             mp.ngroup = (int)cdiv(act, NWAVES);
             mp.nb = mp.nstrip * mp.nchunk * mp.ngroup;
@@ -3052,7 +3057,7 @@ template <typename T> struct ElPlan : ElPlanBase {
             a.A = Ar;
             StrmMap sm;
             sm.nstrip = (int)cdiv(NY + 2, SW_COLS);
-            sm.ch = strm_ch > 0 ? strm_rows_max() : chunk_rows(sm.nstrip, NX + 2, act, 1, STRM_CH);
+            sm.ch = strm_ch > 0 ? strm_rows_max() : adjoint_rows(sm.nstrip, NX + 2, act, sizeof(T));
             sm.nchunk = (int)cdiv(NX + 2, sm.ch);
             sm.ngroup = ng;
             sm.nb = sm.nstrip * sm.nchunk * sm.ngroup;
