@@ -442,6 +442,15 @@ struct AcPlanBase {
         (void)hipGraphExecDestroy(victim->second.exec);
         graphs.erase(victim);
     }
+    // The histories step every shot over all NSTEP levels, so each record has to be that long; the shortest
+    // is the last in plan order.
+    int check_history() const
+    {
+        if (nstep_sorted.back() != p.NSTEP)
+            ADS_FAIL(ADS_ERR_SHAPE, "history mode needs nstep == NSTEP for every shot (shot %lld has %lld of %lld)",
+                     (long long)order.back(), (long long)nstep_sorted.back(), (long long)p.NSTEP);
+        return ADS_OK;
+    }
     virtual ~AcPlanBase()
     {
         drop_graphs();
@@ -1540,8 +1549,7 @@ int ads_acoustic_plan_forward_history(ads_acoustic_plan *plan, const void *model
     clear_error();
     if (!model || !srcv || !u_hist || !scratch) ADS_FAIL(ADS_ERR_ARG, "null argument");
     return dispatch(plan, [&](auto &P) -> int {
-        if (P.NMAX != P.p.NSTEP)
-            ADS_FAIL(ADS_ERR_SHAPE, "history mode needs nstep == NSTEP for every shot");
+        ADS_TRY(P.check_history());
         return P.forward_history(model, srcv, u_hist, phi_hist, psi_hist, scratch, S(stream));
     });
 }
@@ -1555,8 +1563,7 @@ int ads_acoustic_plan_backward_history(ads_acoustic_plan *plan, const void *mode
     if (!model || !srcv || !u_hist || !grad_u_hist || !grad_model || !scratch)
         ADS_FAIL(ADS_ERR_ARG, "null argument");
     return dispatch(plan, [&](auto &P) -> int {
-        if (P.NMAX != P.p.NSTEP)
-            ADS_FAIL(ADS_ERR_SHAPE, "history mode needs nstep == NSTEP for every shot");
+        ADS_TRY(P.check_history());
         return P.backward_history(model, srcv, u_hist, grad_u_hist, grad_model, scratch, S(stream));
     });
 }

@@ -1,0 +1,29 @@
+"""What the full-history entry points ask of a plan, and of the arrays they are given."""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+
+def acoustic_plan(ads, kernel, nstep):
+    p = ads.AcousticPropagatorParams(NX=24, NY=20, NSTEP=max(nstep), DELTAX=10.0, DELTAY=10.0, DELTAT=1e-3,
+                                     NPOINTS_PML=5, vp_ref=2000.0, PropagatorKernel=kernel)
+    w = [1e3 * np.sin(0.3 * np.arange(n)) for n in nstep]
+    srcs = [ads.AcousticSource([8 + 3 * s], [4], v[:, None]) for s, v in enumerate(w)]
+    plan = ads.AcousticPlan(p, srcs, [ads.AcousticReceiver([5], [5])] * len(nstep), dtype=torch.float64, nstep=nstep)
+    c = torch.linspace(1800.0, 2300.0, 26 * 22, dtype=torch.float64, device="cuda").reshape(26, 22)
+    return plan, c, plan.pack_srcv([s.srcv for s in srcs])
+
+
+@pytest.mark.parametrize("kernel", [0, 1])
+@pytest.mark.parametrize("nstep", [[31, 20], [20, 31, 31]])
+def test_acoustic_history_refuses_short_records(ads, cuda, kernel, nstep):
+    """A history holds NSTEP levels of every shot: a plan with a shorter record is refused on the host,
+    whichever shot it is, before anything is written."""
+    plan, c, srcv = acoustic_plan(ads, kernel, nstep)
+    with pytest.raises(Exception, match="nstep == NSTEP"):
+        plan.forward_history(c, srcv)
+    u = torch.zeros((len(nstep), 32, 26, 22), dtype=torch.float64, device="cuda")
+    with pytest.raises(Exception, match="nstep == NSTEP"):
+        plan.backward_history(c, srcv, u, torch.ones_like(u))
