@@ -501,7 +501,6 @@ void ac_fwd_tile(const FwdTile<T> a)
     if (!decode_tile(m, z, s, tile, (int)blockIdx.x)) return;  // workgroup-uniform
     const int4 c = a.tiles[2 * tile], e = a.tiles[2 * tile + 1];
     const int nt = min(a.nt, a.nstep[s] - a.n + 1);
-    if (nt <= 0) return;  // the shot's record ended before this launch (workgroup-uniform)
     LP &lp = *reinterpret_cast<LP *>(raw);
     if (e.w == TILE_PLAIN)
         fwd_tile_body<T, V, RN, VEC, NW, TILE_PLAIN>(a, tile_view<RN, VEC>(c, e), s, tile, nt,
@@ -557,7 +556,6 @@ __device__ inline void adj_tile_body(const AdjTile<T> &a, const TileView &t, int
     const int s1 = min(a.act, (g + 1) * a.Sg);
     for (int s = g * a.Sg; s < s1; s++) {
         const int top = min(a.n, a.nstep[s]);  // a shot enters at its own last level, from zero
-        if (top < m) continue;                 // no level of this shot in the launch (workgroup-uniform)
         const int64_t fo_ = (int64_t)s * a.fstride;
         T A[R][VEC], B[R][VEC], F[R][VEC], G[R][VEC];
 #pragma unroll

@@ -694,8 +694,18 @@ template <typename T> struct AcPlan : AcPlanBase {
         a.srcv_off = d_srcv_off.as<int64_t>();
         a.nsrc = d_nsrc.as<int64_t>();
     }
+    // Each of a launch's first `act` shots has to have the launch's level `lo`, the first that the forward
+    // steps and the last of the adjoint: the kernels count their levels from there on.  Looked at here: one
+    // branch for it in the adjoint tile kernel cost 2 % of a 1000^2 gradient (other scalar spills).
+    int check_levels(int act, int lo) const
+    {
+        if (act < 1 || act > nshots || nstep_sorted[act - 1] < lo)
+            ADS_FAIL(ADS_ERR_SHAPE, "a shot of the launch has no level %d", lo);
+        return ADS_OK;
+    }
     int launch_fwd_tile(FwdTile<T> &a, hipStream_t st)
     {
+        ADS_TRY(check_levels(a.act, a.n));
         a.nb = a.ntiles * a.act;
         const unsigned nb = cdiv(a.nb, NXCD) * NXCD;
         double levels = 0.0;
@@ -710,6 +720,7 @@ template <typename T> struct AcPlan : AcPlanBase {
     // one adjoint launch: levels a.n down to a.n - a.nt + 1
     template <bool DENSE> int launch_adj_tile(AdjTile<T> &a, hipStream_t st)
     {
+        ADS_TRY(check_levels(a.act, a.n - a.nt + 1));
         a.Sg = adj_shape.sg;
         a.nb = a.ntiles * (int)cdiv(a.act, a.Sg);
         const unsigned nb = cdiv(a.nb, NXCD) * NXCD;
