@@ -332,6 +332,14 @@ __global__ void k_model_in(const T *__restrict__ m, T *__restrict__ C, int NX, i
     C[(int64_t)i * P + j] = sq ? v * v : v;
 }
 
+// one dense level of every shot into a history (shot stride hs)
+template <typename T>
+__global__ void k_level_copy(const T *__restrict__ src, T *__restrict__ dst, int64_t hs, int64_t n)
+{
+    const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (q < n) dst[(int64_t)blockIdx.y * hs + q] = src[(int64_t)blockIdx.y * n + q];
+}
+
 // sum of the shot-group accumulators (pitched) -> gradient in caller layout (x 2m if squared)
 template <typename T>
 __global__ void k_grad_out(const T *__restrict__ gC, int64_t stride, int ngroups,
@@ -1034,7 +1042,11 @@ template <typename T> struct AcPlan : AcPlanBase {
                                  (size_t)nshots, st));
         if (phi_hist) ADS_HIP(hipMemsetAsync(phi_hist, 0, H, st));
         if (psi_hist) ADS_HIP(hipMemsetAsync(psi_hist, 0, H, st));
+        // Both auxiliary histories: the tiles write every level into them.  Neither: two scratch buffers of
+        // each, toggled by every launch.  One alone: the buffers with a level per launch, and a copy of the
+        // level (a shot stride of its own for each of the two costs the tile kernel 3 to 5 %: scalar spills).
         const bool aux = phi_hist && psi_hist;
+        T *one = aux ? nullptr : (T *)(phi_hist ? phi_hist : psi_hist);
         if (!aux)
             for (int q = 0; q < 2; q++) {
                 ADS_HIP(hipMemsetAsync(pp[q], 0, F * sizeof(T), st));
@@ -1049,15 +1061,20 @@ template <typename T> struct AcPlan : AcPlanBase {
             a.sstride = hs;
             a.NS = std::numeric_limits<int>::max();
             a.n = (int)n;
-            a.nt = (int)std::min<int64_t>(tile_levels, NMAX - n + 1);
+            a.nt = one ? 1 : (int)std::min<int64_t>(tile_levels, NMAX - n + 1);
             a.phi = aux ? (const T *)phi_hist + (n - 1) * Ndense : pp[set];
             a.psi = aux ? (const T *)psi_hist + (n - 1) * Ndense : qq[set];
             a.phio = aux ? (T *)phi_hist + n * Ndense : pp[set ^ 1];
             a.psio = aux ? (T *)psi_hist + n * Ndense : qq[set ^ 1];
             a.fstride = aux ? hs : Ndense;
             a.plstride = aux ? Ndense : 0;
-            n += a.nt;
             ADS_TRY(launch_fwd_tile(a, st));
+            if (one) {
+                k_level_copy<T><<<dim3(cdiv(Ndense, 256), (unsigned)nshots), 256, 0, st>>>(
+                    phi_hist ? a.phio : a.psio, one + n * Ndense, hs, Ndense);
+                ADS_LAUNCH_CHECK();
+            }
+            n += a.nt;
         }
         return ADS_OK;
     }

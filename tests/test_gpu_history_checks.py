@@ -27,3 +27,21 @@ def test_acoustic_history_refuses_short_records(ads, cuda, kernel, nstep):
     u = torch.zeros((len(nstep), 32, 26, 22), dtype=torch.float64, device="cuda")
     with pytest.raises(Exception, match="nstep == NSTEP"):
         plan.backward_history(c, srcv, u, torch.ones_like(u))
+
+
+@pytest.mark.parametrize("kernel", [0, 1])
+def test_acoustic_history_with_one_auxiliary_array(ads, cuda, kernel):
+    """phi_hist and psi_hist may each be null: whichever is given is filled as when both are."""
+    import ctypes as C
+    plan, c, srcv = acoustic_plan(ads, kernel, [31, 31])
+    ref = plan.forward_history(c, srcv)
+    assert all(float(t.abs().max()) > 0.0 for t in ref)
+    sc = torch.empty(plan.lib.ads_acoustic_plan_history_scratch_size(plan.h), dtype=torch.uint8, device="cuda")
+    st = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    for given in ((True, False), (False, True), (False, False)):
+        out = [torch.full_like(ref[0], 7.0)] + [torch.full_like(ref[0], 7.0) if g else None for g in given]
+        rc = plan.lib.ads_acoustic_plan_forward_history(
+            plan.h, *[None if t is None else C.c_void_p(t.data_ptr()) for t in (c, srcv, *out, sc)], st)
+        assert rc == 0
+        for a, b in zip(out, ref):
+            assert a is None or torch.equal(a, b), given
