@@ -403,7 +403,6 @@ struct AcPlanBase {
     // lies in the rectangle, which is not empty (what ads_acoustic_plan_blocking reports)
     bool blk_ok = false;
     int blocking = 2;
-    int phi_cur = 0;  // buffer that holds phi/psi of the level that the next forward launch starts from
     // tiles of the multi-level kernels (plan and history layout) and their source / receiver lists
     int ntiles = 0;
     DevBuf d_tiles, d_ts_ptr, d_ts_cell, d_ts_ent, d_tr_ptr, d_tr_cell, d_tr_ent;
@@ -525,6 +524,9 @@ template <typename T> struct AcPlan : AcPlanBase {
         T *seg, *phi[2], *psi[2], *P[4], *F[2], *G[2], *gC, *ckpt, *C, *resid;
         double *loss, *part;
         std::vector<size_t> ck_off;  // element offset of each snapshot slot in ckpt
+        // The buffer that holds phi/psi of the level that the next forward launch starts from.  State of one
+        // call, like the rest of this struct: several threads may run a plan, each on its own workspace.
+        int cur = 0;
     };
     int64_t seg_level(const WS &w, int64_t m) const { return std::min<int64_t>(1 + m * w.K, NMAX); }
     int64_t snap_slots(int64_t M, int64_t snaps) const
@@ -649,11 +651,11 @@ template <typename T> struct AcPlan : AcPlanBase {
     }
 
     // one level: the stencil, phi/psi from the new u (kernel 0), sources
-    int fwd_step(const WS &w, int n, const T *srcv, hipStream_t st, const Shape &shape)
+    int fwd_step(WS &w, int n, const T *srcv, hipStream_t st, const Shape &shape)
     {
-        const int act = active[n], cur = phi_cur;
+        const int act = active[n], cur = w.cur;
         if (act <= 0) return ADS_OK;
-        phi_cur ^= 1;
+        w.cur ^= 1;
         FwdArgs<T> a{slot(w, n), cst(slot(w, n - 1)), cst(slot(w, n - 2)), cst(phl(w, cur)), cst(psl(w, cur)),
                      phl(w, cur ^ 1), psl(w, cur ^ 1), w.C, d_sx.as<T>(), d_ty.as<T>(), d_nearx.as<uint8_t>(),
                      d_neary.as<uint8_t>(), (int)NX, (int)NY, (int)Pitch, act, std::min(shape.sg, act), TileMap{}, k};
@@ -672,14 +674,14 @@ template <typename T> struct AcPlan : AcPlanBase {
     }
 
     // forward over levels lo+1..hi from the state held in slots/phi (record traces if asked)
-    int run_forward(const WS &w, int64_t lo, int64_t hi, const T *srcv, T *traces, int record, hipStream_t st,
+    int run_forward(WS &w, int64_t lo, int64_t hi, const T *srcv, T *traces, int record, hipStream_t st,
                     const Shape *sh = nullptr)
     {
         if (sh) return run_forward_levels(w, lo, hi, srcv, traces, record, st, sh);
-        GraphKey key{0, record, phi_cur, lo, hi, w.NS, w.seg, srcv, traces, nullptr};
-        const int end = phi_cur ^ (fwd_launches(lo, hi) & 1);
+        GraphKey key{0, record, w.cur, lo, hi, w.NS, w.seg, srcv, traces, nullptr};
+        const int end = w.cur ^ (fwd_launches(lo, hi) & 1);
         ADS_TRY(replay(key, w.M, st, [&](hipStream_t s) { return run_forward_levels(w, lo, hi, srcv, traces, record, s); }));
-        phi_cur = end;
+        w.cur = end;
         return ADS_OK;
     }
     void tile_common(TileCommon<T> &a, const T *C, int P, int act, const T *srcv) const
@@ -784,7 +786,7 @@ template <typename T> struct AcPlan : AcPlanBase {
         for (int64_t l = lo + 1; l <= hi; l += step) n += active[l] > 0;
         return n;
     }
-    int run_forward_levels(const WS &w, int64_t lo, int64_t hi, const T *srcv, T *traces, int record, hipStream_t st,
+    int run_forward_levels(WS &w, int64_t lo, int64_t hi, const T *srcv, T *traces, int record, hipStream_t st,
                            const Shape *sh = nullptr)
     {
         if (blocking == 1 || sh) {
@@ -800,12 +802,12 @@ template <typename T> struct AcPlan : AcPlanBase {
                 a.NS = (int)w.NS;
                 a.n = (int)n;
                 a.nt = (int)std::min<int64_t>(tile_levels, hi - n + 1);
-                a.phi = w.phi[phi_cur];
-                a.psi = w.psi[phi_cur];
-                a.phio = w.phi[phi_cur ^ 1];
-                a.psio = w.psi[phi_cur ^ 1];
+                a.phi = w.phi[w.cur];
+                a.psi = w.psi[w.cur];
+                a.phio = w.phi[w.cur ^ 1];
+                a.psio = w.psi[w.cur ^ 1];
                 a.fstride = Npad;
-                phi_cur ^= 1;
+                w.cur ^= 1;
                 ADS_TRY(launch_fwd_tile(a, st));
             }
         }
@@ -836,8 +838,8 @@ template <typename T> struct AcPlan : AcPlanBase {
         T *dst = w.ckpt + w.ck_off[q];
         ADS_HIP(hipMemcpyAsync(dst, slot(w, a).p, U * sizeof(T), hipMemcpyDeviceToDevice, st));
         ADS_HIP(hipMemcpyAsync(dst + U, slot(w, a - 1).p, U * sizeof(T), hipMemcpyDeviceToDevice, st));
-        ADS_TRY(frame_copy(false, phl(w, phi_cur), dst + 2 * U, act, st));
-        ADS_TRY(frame_copy(false, psl(w, phi_cur), dst + 2 * U + R, act, st));
+        ADS_TRY(frame_copy(false, phl(w, w.cur), dst + 2 * U, act, st));
+        ADS_TRY(frame_copy(false, psl(w, w.cur), dst + 2 * U + R, act, st));
         return ADS_OK;
     }
 
@@ -851,15 +853,15 @@ template <typename T> struct AcPlan : AcPlanBase {
         if (q < 0) {
             ADS_HIP(hipMemsetAsync(slot(w, 0).p, 0, U * sizeof(T), st));
             ADS_HIP(hipMemsetAsync(slot(w, 1).p, 0, U * sizeof(T), st));
-            ADS_HIP(hipMemsetAsync(phl(w, phi_cur).p, 0, U * sizeof(T), st));
-            ADS_HIP(hipMemsetAsync(psl(w, phi_cur).p, 0, U * sizeof(T), st));
+            ADS_HIP(hipMemsetAsync(phl(w, w.cur).p, 0, U * sizeof(T), st));
+            ADS_HIP(hipMemsetAsync(psl(w, w.cur).p, 0, U * sizeof(T), st));
             return ADS_OK;
         }
         const T *src = w.ckpt + w.ck_off[q];
         ADS_HIP(hipMemcpyAsync(slot(w, a).p, src, U * sizeof(T), hipMemcpyDeviceToDevice, st));
         ADS_HIP(hipMemcpyAsync(slot(w, a - 1).p, src + U, U * sizeof(T), hipMemcpyDeviceToDevice, st));
-        ADS_TRY(frame_copy(true, phl(w, phi_cur), const_cast<T *>(src) + 2 * U, act, st));
-        ADS_TRY(frame_copy(true, psl(w, phi_cur), const_cast<T *>(src) + 2 * U + R, act, st));
+        ADS_TRY(frame_copy(true, phl(w, w.cur), const_cast<T *>(src) + 2 * U, act, st));
+        ADS_TRY(frame_copy(true, psl(w, w.cur), const_cast<T *>(src) + 2 * U + R, act, st));
         return ADS_OK;
     }
 
@@ -881,7 +883,6 @@ template <typename T> struct AcPlan : AcPlanBase {
         ADS_TRY(prepare_C(w.C, model, (int)Pitch, st));
         ADS_HIP(hipMemsetAsync(slot(w, 0).p, 0, F, st));
         ADS_HIP(hipMemsetAsync(slot(w, 1).p, 0, F, st));
-        phi_cur = 0;
         for (int q = 0; q < 2; q++) {
             ADS_HIP(hipMemsetAsync(w.phi[q], 0, F, st));
             ADS_HIP(hipMemsetAsync(w.psi[q], 0, F, st));
@@ -920,7 +921,7 @@ template <typename T> struct AcPlan : AcPlanBase {
         const T *sv = (const T *)srcv;
         struct Ops {
             AcPlan *pl;
-            const WS &w;
+            WS &w;
             const T *sv, *resid;
             hipStream_t st;
             int set;  // state set of the next adjoint launch
@@ -972,7 +973,6 @@ template <typename T> struct AcPlan : AcPlanBase {
         ADS_TRY(prepare_C(w.C, model, (int)Pitch, st));
         const size_t F = (size_t)nshots * Npad * sizeof(T);
         for (int64_t q = 0; q < std::min<int64_t>(w.NS, 4); q++) ADS_HIP(hipMemsetAsync(slot(w, q).p, 0, F, st));
-        phi_cur = 0;
         for (int q = 0; q < 2; q++) {
             ADS_HIP(hipMemsetAsync(w.phi[q], 0, F, st));
             ADS_HIP(hipMemsetAsync(w.psi[q], 0, F, st));
