@@ -413,11 +413,12 @@ struct AcPlanBase {
     struct GraphKey {
         int kind, record, set;  // set: the phi/psi buffer or adjoint state set that the segment starts from
         int64_t lo, hi, ns;  // ns: slots of the workspace layout (fixes every slot address)
-        const void *ws, *srcv, *traces, *resid;
+        // model: the workspace's C, which lies behind the checkpoints and so moves with the snapshot count
+        const void *ws, *model, *srcv, *traces, *resid;
         bool operator<(const GraphKey &o) const
         {
-            return std::tie(kind, record, set, lo, hi, ns, ws, srcv, traces, resid) <
-                   std::tie(o.kind, o.record, o.set, o.lo, o.hi, o.ns, o.ws, o.srcv, o.traces, o.resid);
+            return std::tie(kind, record, set, lo, hi, ns, ws, model, srcv, traces, resid) <
+                   std::tie(o.kind, o.record, o.set, o.lo, o.hi, o.ns, o.ws, o.model, o.srcv, o.traces, o.resid);
         }
     };
     // A cached graph also records its last use: the key holds the caller's trace / residual
@@ -678,7 +679,7 @@ template <typename T> struct AcPlan : AcPlanBase {
                     const Shape *sh = nullptr)
     {
         if (sh) return run_forward_levels(w, lo, hi, srcv, traces, record, st, sh);
-        GraphKey key{0, record, w.cur, lo, hi, w.NS, w.seg, srcv, traces, nullptr};
+        GraphKey key{0, record, w.cur, lo, hi, w.NS, w.seg, w.C, srcv, traces, nullptr};
         const int end = w.cur ^ (fwd_launches(lo, hi) & 1);
         ADS_TRY(replay(key, w.M, st, [&](hipStream_t s) { return run_forward_levels(w, lo, hi, srcv, traces, record, s); }));
         w.cur = end;
@@ -936,7 +937,7 @@ template <typename T> struct AcPlan : AcPlanBase {
             int adjoint(int64_t m)
             {
                 const int64_t a = pl->seg_level(w, m), b = pl->seg_level(w, m + 1);
-                GraphKey key{1, 0, set, a, b, w.NS, w.seg, sv, nullptr, resid};
+                GraphKey key{1, 0, set, a, b, w.NS, w.seg, w.C, sv, nullptr, resid};
                 ADS_TRY(pl->replay(key, w.M, st, [&](hipStream_t s) { return pl->adj_levels(w, a, b, set, sv, resid, s); }));
                 set ^= pl->adj_launches(a, b) & 1;
                 return ADS_OK;

@@ -1,7 +1,8 @@
-"""A plan holds no state of a call in flight."""
+"""A plan holds no state of a call in flight, and a replayed graph belongs to the buffers of its call."""
 import ctypes as C
 import threading
 
+import numpy as np
 import pytest
 
 from test_gpu_acoustic import T, make_case
@@ -44,3 +45,37 @@ def test_two_threads_share_a_plan(orc, ads, cuda, kernel):
         t.join()
     torch.cuda.synchronize()
     assert not bad, bad
+
+
+@pytest.mark.parametrize("kernel", [0, 1])
+def test_graphs_follow_the_snapshot_count(orc, ads, cuda, kernel):
+    """The snapshot count moves the arrays behind the checkpoints within an unchanged workspace buffer: with
+    graphs on, a gradient after fewer snapshots and for another model equals the one without graphs, bit
+    for bit, and again when the first count returns."""
+    p, c, srcs, rcvs, nstep = make_case(orc, ads, NX=40, NY=36, NSTEP=90, npml=8, nshots=2, kernel=kernel, seed=6)
+    plan = ads.AcousticPlan(p, srcs, rcvs, dtype=torch.float64, nstep=nstep)
+    srcv, K = plan.pack_srcv([s.srcv for s in srcs]), 8
+    tr = torch.empty(plan.trace_elems, dtype=torch.float64, device="cuda")
+    cot = T(np.random.default_rng(1).standard_normal(plan.trace_elems))
+    ws = torch.empty(plan.workspace_size(K), dtype=torch.uint8, device="cuda")  # one-level: the largest
+    st = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    P = lambda t: C.c_void_p(t.data_ptr())
+
+    def pullback(m):
+        g = torch.empty_like(m)
+        assert plan.lib.ads_acoustic_plan_forward(plan.h, P(m), P(srcv), P(tr), P(ws), ws.numel(), K, st) == 0
+        assert plan.lib.ads_acoustic_plan_backward(plan.h, P(m), P(srcv), P(cot), P(g), P(ws), ws.numel(), K, st) == 0
+        torch.cuda.synchronize()
+        return g
+
+    steps = [(-1, T(c)), (2, T(0.93 * c)), (0, T(1.04 * c)), (-1, T(0.97 * c))]
+    want = []
+    for S, m in steps:
+        plan.set_snapshots(S)
+        want.append(pullback(m))
+    plan.set_graph(True)
+    for (S, m), w in zip(steps, want):
+        plan.set_snapshots(S)
+        for _ in range(3):
+            assert torch.equal(pullback(m), w), S
+    plan.set_graph(False)
