@@ -2624,6 +2624,15 @@ struct ElPlanBase {
     int64_t snapshots = -1;
     int sub = 0;          // one MPIElastic subdomain (see ElCoef)
     int64_t PX = 0, PY = 0;  // CPML profile lengths (NX, NY; the block size in the subdomain form)
+    // The histories and their cotangents hold NSTEP levels of every shot; the shortest record is the last in
+    // plan order.
+    int check_history(const char *what) const
+    {
+        if (nstep_sorted.back() != p.NSTEP)
+            ADS_FAIL(ADS_ERR_SHAPE, "%s nstep == NSTEP for every shot (shot %lld has %lld of %lld)", what,
+                     (long long)order.back(), (long long)nstep_sorted.back(), (long long)p.NSTEP);
+        return ADS_OK;
+    }
 };
 
 template <typename T> struct ElPlan : ElPlanBase {
@@ -3681,7 +3690,7 @@ int ads_elastic_plan_backward_dense(ads_elastic_plan *plan, const void *rho, con
     if (!rho || !lam || !mu || !srcv || !grad_hist || !grad_rho || !grad_lam || !grad_mu)
         ADS_FAIL(ADS_ERR_ARG, "null argument");
     return el_dispatch(plan, [&](auto &P) -> int {
-        if (P.NMAX != P.p.NSTEP) ADS_FAIL(ADS_ERR_SHAPE, "dense cotangents need nstep == NSTEP for every shot");
+        ADS_TRY(P.check_history("dense cotangents need"));
         ADS_TRY(P.forward(rho, lam, mu, srcv, nullptr, ws, wsb, K, S(stream), true));
         return P.backward(srcv, nullptr, grad_hist, grad_rho, grad_lam, grad_mu, ws, wsb, K, S(stream));
     });
@@ -3701,7 +3710,7 @@ int ads_elastic_forward_history(ads_elastic_plan *plan, const void *rho, const v
     clear_error();
     if (!rho || !lam || !mu || !srcv || !hist || !scratch) ADS_FAIL(ADS_ERR_ARG, "null argument");
     return el_dispatch(plan, [&](auto &P) -> int {
-        if (P.NMAX != P.p.NSTEP) ADS_FAIL(ADS_ERR_SHAPE, "history mode needs nstep == NSTEP for every shot");
+        ADS_TRY(P.check_history("history mode needs"));
         return P.forward_history(rho, lam, mu, srcv, hist, scratch, S(stream));
     });
 }

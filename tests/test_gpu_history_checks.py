@@ -45,3 +45,18 @@ def test_acoustic_history_with_one_auxiliary_array(ads, cuda, kernel):
         assert rc == 0
         for a, b in zip(out, ref):
             assert a is None or torch.equal(a, b), given
+
+
+@pytest.mark.parametrize("nstep", [[24, 15], [15, 24, 24]])
+def test_elastic_history_refuses_short_records(ads, cuda, nstep):
+    """As the acoustic calls: the history and the pullback of a dense cotangent."""
+    p = ads.ElasticPropagatorParams(NX=24, NY=20, NSTEP=max(nstep), DELTAX=10.0, DELTAY=10.0, DELTAT=1e-3,
+                                    NPOINTS_PML=5, vp_ref=2500.0, f0=8.0)
+    srcs = [ads.ElasticSource([8, 8], [6, 6], [2, 3], np.ones((n, 2))) for n in nstep]
+    plan = ads.ElasticPlan(p, srcs, [ads.ElasticReceiver([5], [5], [0])] * len(nstep), dtype=torch.float64, nstep=nstep)
+    srcv = plan.pack_srcv([s.srcv for s in srcs])
+    m = [torch.full((26, 22), v, dtype=torch.float64, device="cuda") for v in (2000.0, 4e9, 4e9)]
+    with pytest.raises(Exception, match="nstep == NSTEP"):
+        plan.forward_history(*m, srcv)
+    with pytest.raises(Exception, match="nstep == NSTEP"):
+        plan.backward_dense(*m, srcv, torch.ones((len(nstep), 5, 25, 26, 22), dtype=torch.float64, device="cuda"), 8)
