@@ -732,7 +732,7 @@ template <typename T> struct AcPlan : AcPlanBase {
     template <bool DENSE> int launch_adj_tile(AdjTile<T> &a, hipStream_t st)
     {
         ADS_TRY(check_levels(a.act, a.n - a.nt + 1));
-        a.Sg = adj_shape.sg;
+        a.Sg = std::min(adj_shape.sg, a.act);  // (any count is accepted; the kernel adds it to act)
         a.nb = a.ntiles * (int)cdiv(a.act, a.Sg);
         const unsigned nb = cdiv(a.nb, NXCD) * NXCD;
         double levels = 0.0;

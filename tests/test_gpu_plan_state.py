@@ -1,4 +1,5 @@
-"""A plan holds no state of a call in flight, and a replayed graph belongs to the buffers of its call."""
+"""A plan holds no state of a call in flight, a replayed graph belongs to the buffers of its call, and the
+settings of a plan hold over their whole range."""
 import ctypes as C
 import threading
 
@@ -79,3 +80,16 @@ def test_graphs_follow_the_snapshot_count(orc, ads, cuda, kernel):
         for _ in range(3):
             assert torch.equal(pullback(m), w), S
     plan.set_graph(False)
+
+
+def test_shots_per_adjoint_workgroup_up_to_the_largest_int(orc, ads, cuda):
+    """set_shape takes any positive number of shots per workgroup; more than the plan has mean all of them."""
+    p, c, srcs, rcvs, nstep = make_case(orc, ads, NX=40, NY=36, NSTEP=60, npml=8, nshots=3, kernel=1, seed=7, uneven=True)
+    plan = ads.AcousticPlan(p, srcs, rcvs, dtype=torch.float64, nstep=nstep)
+    srcv = plan.pack_srcv([s.srcv for s in srcs])
+    obs = plan.forward(T(1.03 * c), srcv, 9).clone()
+    out = []
+    for sg in (3, 4, 2**31 - 1):
+        plan.set_shape((2, sg, 1, 2, sg, 1))
+        out.append(plan.gradient(T(c), srcv, obs, 9)[1].clone())
+    assert torch.equal(out[1], out[0]) and torch.equal(out[2], out[0])
