@@ -102,7 +102,9 @@ __device__ inline T ac_pml_num(const AcCoef<T> &k, T a2, T e, T wc, T wold, T C,
     return a2 * wc + C * lap + k.ex * dphi + k.ey * dpsi - e * wold;
 }
 // phi^n = (1 - dt sigma) phi + C (tau - sigma) fx dv, psi^n = (1 - dt tau) psi - C (tau - sigma) fy dv;
-// d1 the damping factor, ct = C (tau - sigma)
+// d1 the damping factor, ct = C (tau - sigma).  Taken where ct != 0 only: elsewhere phi and psi stay the 0 that
+// they start from, also beside a dv that is not finite.  (In the tiles the comparison costs no register
+// over the levels and no time; the flags "interior" and "in the PML" cost up to 2.6 %.)
 template <typename T> __device__ inline T ac_phi(const AcCoef<T> &k, T d1, T phi, T ct, T dv)
 {
     return d1 * phi + ct * k.fx * dv;
@@ -428,8 +430,12 @@ __device__ inline void fwd_tile_body(const FwdTile<T> &a, const TileView &t, int
                     Y[r][e] = pc.in(r, e) ? out : T(0);
                     if constexpr (V == 1) {
                         const T ct = C[r][e] * pc.c(r, e);
-                        F_[e] = ac_phi(k, pc.d1(r), F[r][e], ct, ws - wn);
-                        G_[e] = ac_psi(k, pc.tk[e], G[r][e], ct, we - ww);
+                        F_[e] = F[r][e];
+                        G_[e] = G[r][e];
+                        if (ct != T(0)) {
+                            F_[e] = ac_phi(k, pc.d1(r), F[r][e], ct, ws - wn);
+                            G_[e] = ac_psi(k, pc.tk[e], G[r][e], ct, we - ww);
+                        }
                     }
                     fn[e] = F[r][e];
                 }
@@ -455,9 +461,12 @@ __device__ inline void fwd_tile_body(const FwdTile<T> &a, const TileView &t, int
                 for (int e = 0; e < VEC; e++) {
                     const T vn = r > 0 ? Y[r > 0 ? r - 1 : r][e] : vn_[e];
                     const T vs = r < R - 1 ? Y[r < R - 1 ? r + 1 : r][e] : vs_[e];
+                    const T ve = east_of(Y[r], e), vw = west_of(Y[r], e);  // (by every lane)
                     const T ct = C[r][e] * pc.c(r, e);
-                    F[r][e] = ac_phi(k, pc.d1(r), F[r][e], ct, vs - vn);
-                    G[r][e] = ac_psi(k, pc.tk[e], G[r][e], ct, east_of(Y[r], e) - west_of(Y[r], e));
+                    if (ct != T(0)) {
+                        F[r][e] = ac_phi(k, pc.d1(r), F[r][e], ct, vs - vn);
+                        G[r][e] = ac_psi(k, pc.tk[e], G[r][e], ct, ve - vw);
+                    }
                 }
         }
         // the next level's value is loaded inside the same branch: a load carried to the loop's end
