@@ -513,9 +513,11 @@ template <typename T> struct AcPlan : AcPlanBase {
         else launch_level<2, 1>(a, st);
     }
 
-    double fwd_level_bytes(int act) const
+    // What a launch has to move, for the profile: one value per interior cell and shot
+    double cell_bytes() const { return (double)NX * (double)NY * sizeof(T); }
+    double fwd_level_bytes(int act) const  // single-level forward
     {
-        return (double)act * (double)NX * (double)NY * sizeof(T) * (4.0 + (variant == 1 ? 4.0 : 2.0) * f_pml);
+        return (double)act * cell_bytes() * (4.0 + (variant == 1 ? 4.0 : 2.0) * f_pml);
     }
     int64_t group_arrays() const { return (int64_t)cdiv(nshots, adj_shape.sg); }
 
@@ -725,7 +727,8 @@ template <typename T> struct AcPlan : AcPlanBase {
         int pr = prof_start(ADS_PROF_AC_FWD, st);
         if (variant == 1) ac_fwd_tile<T, 1, TILE_RN, TILE_RP, 1, TILE_WAVES><<<nb, TILE_WAVES * WAVE, 0, st>>>(a);
         else ac_fwd_tile<T, 0, TILE_RN, TILE_RP, 1, TILE_WAVES><<<nb, TILE_WAVES * WAVE, 0, st>>>(a);
-        prof_stop(pr, st, fwd_level_bytes(1) * levels, a.nt);
+        // per launch: u^{n-1}, u^{n-2}, C and phi/psi once, phi/psi back once, every level's u
+        prof_stop(pr, st, cell_bytes() * (levels + a.act * (3.0 + 4.0 * f_pml)), a.nt);
         ADS_LAUNCH_CHECK();
         return ADS_OK;
     }
@@ -741,7 +744,10 @@ template <typename T> struct AcPlan : AcPlanBase {
         int pr = prof_start(ADS_PROF_AC_ADJ, st);
         if (variant == 1) ac_adj_tile<T, 1, TILE_RN, TILE_RP, 1, TILE_WAVES, DENSE><<<nb, TILE_WAVES * WAVE, 0, st>>>(a);
         else ac_adj_tile<T, 0, TILE_RN, TILE_RP, 1, TILE_WAVES, DENSE><<<nb, TILE_WAVES * WAVE, 0, st>>>(a);
-        prof_stop(pr, st, (double)NX * (double)NY * sizeof(T) * (7.0 + (variant == 1 ? 4.0 : 2.0) * f_pml) * levels, a.nt);
+        // per launch: P^{n+1}, P^{n+2} and F/G in and out, C and dL/dC in and out once per group of shots, and
+        // every level's u (kernel 0's PML: one more) and dense cotangent
+        const double per_shot = 4.0 + (variant == 1 ? 4.0 : 5.0) * f_pml;
+        prof_stop(pr, st, cell_bytes() * ((DENSE ? 2.0 : 1.0) * levels + a.act * per_shot + 3.0 * cdiv(a.act, a.Sg)), a.nt);
         ADS_LAUNCH_CHECK();
         return ADS_OK;
     }

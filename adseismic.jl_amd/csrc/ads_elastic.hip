@@ -2944,7 +2944,10 @@ template <typename T> struct ElPlan : ElPlanBase {
         const int pr = prof_start(ADS_PROF_EL_FWD_STRESS, st);
         if (sub) el_fwd_tile<T, 1, TILE_R><<<nb, WAVE * ET_NW, 0, st>>>(a);
         else el_fwd_tile<T, 0, TILE_R><<<nb, WAVE * ET_NW, 0, st>>>(a);
-        prof_stop(pr, st, (double)act * PX * PY * nt * sizeof(T) * (13.0 + 8.0 * f_x + 8.0 * f_y), nt);
+        // per launch: the fields, parameters and memory variables in once, the fields of every level out, the
+        // memory variables with them (histories: once)
+        const double mv = 4.0 * f_x + 4.0 * f_y;
+        prof_stop(pr, st, (double)act * PX * PY * sizeof(T) * (8.0 + 5.0 * nt + mv * (a.mo ? 2 : 1 + nt)), nt);
         ADS_LAUNCH_CHECK();
         return ADS_OK;
     }

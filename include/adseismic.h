@@ -415,14 +415,21 @@ int ads_elastic_forward_history(ads_elastic_plan *plan, const void *rho, const v
  * Kernel timing for benchmarks.  Between ads_profile_begin() and ads_profile_end() every
  * launch of the main stencil kernels made by the plan entry points is bracketed by HIP events
  * on its launch stream; ads_profile_end() waits for them and accumulates, per kernel class,
- * the summed duration, the launch count and the algorithmic HBM bytes of those launches
- * (compulsory per-cell traffic: acoustic forward w(4 + 4 f_pml), adjoint w(7 + 4 f_pml) for
- * PropagatorKernel 1, w(4 + 2 f_pml) and w(7 + 2 f_pml) for kernel 0; elastic forward w(8 + 4 f_x + 4 f_y) stress and w(5 + 4 f_x + 4 f_y)
- * velocity phase, adjoint w(12 + 4 f_x + 4 f_y) per phase: the whole-step counts
- * w(13 + 8 f_x + 8 f_y) and w(24 + 8 f_x + 8 f_y) split by the fields each phase updates; the
- * fused elastic forward step, the default, is timed in ADS_PROF_EL_FWD_STRESS with the
- * whole-step count and leaves ADS_PROF_EL_FWD_VEL empty).  A launch that advances several time
- * levels (the acoustic tiles) counts as that many launches.
+ * the summed duration, the launch count and the algorithmic HBM bytes of those launches: what
+ * they have to move, with w bytes per value and cell and with f_pml, f_x, f_y the interior
+ * fractions inside the PML strips.
+ *   Acoustic tiles, nt levels per launch: forward w(nt + 3 + 4 f_pml) per shot; adjoint
+ *   w(nt + 4 + 4 f_pml) per shot (PropagatorKernel 0: 5 f_pml; dense cotangent: 2 nt) and 3 w per
+ *   group of shots.  Single-level forward (set_blocking(1)): w(4 + 4 f_pml), kernel 0 w(4 + 2 f_pml)
+ *   without its phi/psi pass.
+ *   Elastic, one level per launch: forward w(8 + 4 f_x + 4 f_y) stress and w(5 + 4 f_x + 4 f_y)
+ *   velocity phase, adjoint w(12 + 4 f_x + 4 f_y) per phase: the whole-step counts
+ *   w(13 + 8 f_x + 8 f_y) and w(24 + 8 f_x + 8 f_y) split by the fields each phase updates.  The
+ *   fused forward step (FP32 plans) is timed in ADS_PROF_EL_FWD_STRESS with the whole-step count
+ *   and leaves ADS_PROF_EL_FWD_VEL empty; so are the elastic tiles (FP64 plans, dense histories),
+ *   nt levels per launch, with w(8 + 5 nt + (1 + nt)(4 f_x + 4 f_y)).
+ * A launch that advances several time levels (the tiles of both schemes) counts as that many
+ * launches.
  * ads_profile_begin_sampled(every) brackets only launches 0, every, 2*every, ... of each class
  * (counted from the begin call), so that a long timed run carries few events; the queried
  * duration, launch count and bytes then cover those launches alone.  ads_profile_begin() is
