@@ -114,6 +114,11 @@ template <typename T> __device__ inline T ac_psi(const AcCoef<T> &k, T d1, T psi
     return d1 * psi - ct * k.fy * dv;
 }
 
+// Columns per lane.  The kernels' register arrays have this last dimension, of 1, only because their code comes
+// out better with it: without it the same expressions take other registers and scalar spills, and the adjoint is
+// slower (517 x 389, 6 shots, FP32 gradient 7.18 -> 7.43 ms; 200 x 66, 8 shots, FP64 15.5 -> 15.7 ms).
+constexpr int VEC = 1;
+
 // A tile as one wavefront sees it.
 struct TileView {
     int i0, i1, j0, j1;  // core
@@ -123,7 +128,7 @@ struct TileView {
                          // beyond the extent repeats its edge and is never stored
     int jend;            // one past the extent's last column
 };
-template <int R, int VEC> __device__ inline TileView tile_view(const int4 c, const int4 e)
+template <int R> __device__ inline TileView tile_view(const int4 c, const int4 e)
 {
     TileView v;
     v.i0 = c.x, v.i1 = c.y, v.j0 = c.z, v.j1 = c.w;
@@ -132,49 +137,33 @@ template <int R, int VEC> __device__ inline TileView tile_view(const int4 c, con
     const int ne = e.z & 0xffff, ce = e.z >> 16;
     v.r0 = e.x + v.w * R;
     v.nr = min(max(ne - v.w * R, 0), R);
-    v.j = e.y + v.lane * VEC;
-    v.jc = e.y + min(v.lane, (ce - 1) / VEC) * VEC;
+    v.j = e.y + v.lane;
+    v.jc = e.y + min(v.lane, ce - 1);
     v.last = e.x + ne - 1;
     v.jend = e.y + ce;
     return v;
 }
-// east / west neighbour of column e of a lane's VEC columns
-template <typename T, int VEC> __device__ inline T east_of(const T (&x)[VEC], int e)
-{
-    return e < VEC - 1 ? x[e < VEC - 1 ? e + 1 : e] : lane_east(x[0]);
-}
-template <typename T, int VEC> __device__ inline T west_of(const T (&x)[VEC], int e)
-{
-    return e > 0 ? x[e > 0 ? e - 1 : e] : lane_west(x[VEC - 1]);
-}
-// Stores rows r of x whose bit is set in `rows` (wave-uniform) and columns [j0, j1) of the lane's VEC
-// columns from j; ro: byte offset of each row (wave-uniform), jb of the lane's column.
-template <typename T, int R, int VEC>
+// Stores rows r of x whose bit is set in `rows` (wave-uniform) from the lanes whose column j lies in
+// [j0, j1); ro: byte offset of each row (wave-uniform), jb of the lane's column.
+template <typename T, int R>
 __device__ inline void store_rows(T *base, const uint32_t *ro, uint32_t jb, const T (&x)[R][VEC], uint32_t rows, int j,
                                   int j0, int j1)
 {
-    if (j >= j0 && j + VEC <= j1) {
-        if (rows == (1u << R) - 1) {
+    if (j < j0 || j >= j1) return;
+    if (rows == (1u << R) - 1) {
 #pragma unroll
-            for (int r = 0; r < R; r++) vst(at_off(at_off(base, ro[r]), jb), x[r]);
-        } else {
-#pragma unroll
-            for (int r = 0; r < R; r++)
-                if (rows >> r & 1) vst(at_off(at_off(base, ro[r]), jb), x[r]);
-        }
-    } else if (VEC > 1 && j < j1 && j + VEC > j0) {
+        for (int r = 0; r < R; r++) vst(at_off(at_off(base, ro[r]), jb), x[r]);
+    } else {
 #pragma unroll
         for (int r = 0; r < R; r++)
-#pragma unroll
-            for (int e = 0; e < VEC; e++)
-                if ((rows >> r & 1) && j + e >= j0 && j + e < j1) at_off(at_off(base, ro[r]), jb)[e] = x[r][e];
+            if (rows >> r & 1) vst(at_off(at_off(base, ro[r]), jb), x[r]);
     }
 }
 
 // PML coefficients of a lane's cells.  sg: sigma per row (scalars).  TILE_X: e, 1 + h, its reciprocal and d1
 // per row (scalars); TILE_Y: the same per column; TILE_XY: the reciprocal per cell, the rest formed where it
 // is used.
-template <typename T, int R, int VEC, int KIND> struct PmlCoef {
+template <typename T, int R, int KIND> struct PmlCoef {
     static constexpr bool X = KIND == TILE_X, Y = KIND == TILE_Y, XY = KIND == TILE_XY;
     T sg[R], re[X ? R : 1], rh[X ? R : 1], ri[X ? R : 1], rd[X || XY ? R : 1];
     T tu[VEC], te[Y ? VEC : 1], th[Y ? VEC : 1], ti[Y ? VEC : 1], tk[VEC], inv[XY ? R : 1][VEC];
@@ -184,11 +173,11 @@ template <typename T, int R, int VEC, int KIND> struct PmlCoef {
     {
 #pragma unroll
         for (int e = 0; e < VEC; e++) {
-            const bool cok = t.j + e < t.jend;
-            jin[e] = t.j + e >= 1 && t.j + e <= a.NY && cok;
-            tu[e] = !X && cok ? a.ty[t.j + e] : T(0);
+            const bool cok = t.j < t.jend;
+            jin[e] = t.j >= 1 && t.j <= a.NY && cok;
+            tu[e] = !X && cok ? a.ty[t.j] : T(0);
             tk[e] = T(1) - k.dt * tu[e];
-            ny[e] = !X && cok && a.neary[t.j + e] != 0;
+            ny[e] = !X && cok && a.neary[t.j] != 0;
             if constexpr (Y) {
                 te[e] = T(1) - tu[e] * k.hdt;
                 th[e] = T(1) + tu[e] * k.hdt;
@@ -273,9 +262,9 @@ __device__ inline WavePoints wave_points(const PointList &p, int64_t at, int row
 
 // Adds dt^2 srcv[lev - 1, .] at the wavefront's source cells to rows of B, entry by entry in
 // source order (Core.jl:593-601).  `first`: the value of the lane's own first cell and entry.
-template <typename T, int R, int VEC>
+template <typename T, int R>
 __device__ inline void add_points(const TileCommon<T> &a, const WavePoints &wp, int row0, int lane,
-                                  T (*__restrict__ plane)[WAVE * VEC], const T *__restrict__ srow, T first,
+                                  T (*__restrict__ plane)[WAVE], const T *__restrict__ srow, T first,
                                   T (&B)[R][VEC])
 {
     for (int k = 0;; k++) {
@@ -294,8 +283,8 @@ __device__ inline void add_points(const TileCommon<T> &a, const WavePoints &wp, 
             if (wp.rows >> r & 1) {  // uniform
 #pragma unroll
                 for (int e = 0; e < VEC; e++) {
-                    B[r][e] += plane[r][lane * VEC + e];
-                    plane[r][lane * VEC + e] = T(0);
+                    B[r][e] += plane[r][lane];
+                    plane[r][lane] = T(0);
                 }
             }
         __builtin_amdgcn_wave_barrier();
@@ -326,25 +315,25 @@ __device__ inline void sum_points(const PointList &p, const WavePoints &wp, int 
 // ---------------------------------------------------------------------------------------------
 // forward
 // ---------------------------------------------------------------------------------------------
-template <typename T, int V, int R, int VEC, int NW, bool PML> struct FwdTileLds {
-    T u[2][NW][2][WAVE * VEC];
-    T p[PML ? 2 : 0][NW][2][WAVE * VEC];            // phi rows
-    T v[PML && V == 0 ? 2 : 0][NW][2][WAVE * VEC];  // u^n before the sources
-    T plane[NW][R][WAVE * VEC];
+template <typename T, int V, int R, int NW, bool PML> struct FwdTileLds {
+    T u[2][NW][2][WAVE];
+    T p[PML ? 2 : 0][NW][2][WAVE];            // phi rows
+    T v[PML && V == 0 ? 2 : 0][NW][2][WAVE];  // u^n before the sources
+    T plane[NW][R][WAVE];
 };
 
-template <typename T, int V, int R, int VEC, int NW, int KIND>
+template <typename T, int V, int R, int NW, int KIND>
 __device__ inline void fwd_tile_body(const FwdTile<T> &a, const TileView &t, int s, int tile, int nt,
-                                     FwdTileLds<T, V, R, VEC, NW, KIND != TILE_PLAIN> &lds)
+                                     FwdTileLds<T, V, R, NW, KIND != TILE_PLAIN> &lds)
 {
     constexpr bool PML = KIND != TILE_PLAIN;
     const AcCoef<T> k = a.k;
-    const int lane = t.lane, w = t.w, j = t.j, lv = lane * VEC;
+    const int lane = t.lane, w = t.w, j = t.j;
     const uint32_t jb = (uint32_t)j * (uint32_t)sizeof(T), jcb = (uint32_t)t.jc * (uint32_t)sizeof(T);
     const int lrow = w * R;  // first register row within the extent
     const T zero[VEC] = {};
 #pragma unroll
-    for (int r = 0; r < R; r++) vst(&lds.plane[w][r][lv], zero);
+    for (int r = 0; r < R; r++) vst(&lds.plane[w][r][lane], zero);
     uint32_t ro[R];  // byte offset of each row, clamped to the extent (wave-uniform)
 #pragma unroll
     for (int r = 0; r < R; r++) ro[r] = (uint32_t)min(t.r0 + r, t.last) * ((uint32_t)a.P * (uint32_t)sizeof(T));
@@ -376,7 +365,7 @@ __device__ inline void fwd_tile_body(const FwdTile<T> &a, const TileView &t, int
     const int64_t ns = a.nsrc[s];
     const T *__restrict__ srow = a.srcv + a.srcv_off[s] + (int64_t)(a.n - 1) * ns;
     T pv = first_point(a.src, wp, lane, srow);
-    PmlCoef<T, R, VEC, KIND> pc;
+    PmlCoef<T, R, KIND> pc;
     if constexpr (PML) {
         pc.load(t, a, k);
 #pragma unroll
@@ -393,20 +382,20 @@ __device__ inline void fwd_tile_body(const FwdTile<T> &a, const TileView &t, int
                 for (int r = 0; r < R; r++) recompute(C[r][e]);
             }
         }
-        vst(&lds.u[par][w][0][lv], X[0]);
-        vst(&lds.u[par][w][1][lv], X[R - 1]);
+        vst(&lds.u[par][w][0][lane], X[0]);
+        vst(&lds.u[par][w][1][lane], X[R - 1]);
         if constexpr (PML) {
-            vst(&lds.p[par][w][0][lv], F[0]);
-            vst(&lds.p[par][w][1][lv], F[R - 1]);
+            vst(&lds.p[par][w][0][lane], F[0]);
+            vst(&lds.p[par][w][1][lane], F[R - 1]);
         }
         __syncthreads();
         // rows r0 - 1 and r0 + R (beyond the tile's first and last row: any value)
         T un_[VEC], us_[VEC], fn[VEC], fs_[VEC];
-        vld(un_, &lds.u[par][wu][1][lv]);
-        vld(us_, &lds.u[par][wd][0][lv]);
+        vld(un_, &lds.u[par][wu][1][lane]);
+        vld(us_, &lds.u[par][wd][0][lane]);
         if constexpr (PML) {
-            vld(fn, &lds.p[par][wu][1][lv]);
-            vld(fs_, &lds.p[par][wd][0][lv]);
+            vld(fn, &lds.p[par][wu][1][lane]);
+            vld(fs_, &lds.p[par][wd][0][lane]);
         }
 #pragma unroll
         for (int r = 0; r < R; r++) {
@@ -415,7 +404,7 @@ __device__ inline void fwd_tile_body(const FwdTile<T> &a, const TileView &t, int
             for (int e = 0; e < VEC; e++) {
                 const T wc = X[r][e], wn = r > 0 ? X[r > 0 ? r - 1 : r][e] : un_[e];
                 const T ws = r < R - 1 ? X[r < R - 1 ? r + 1 : r][e] : us_[e];
-                const T we = east_of(X[r], e), ww = west_of(X[r], e);
+                const T we = lane_east(X[r][e]), ww = lane_west(X[r][e]);
                 const T lap = ac_lap(k, wc, ws, wn, we, ww);
                 if constexpr (!PML) {
                     Y[r][e] = ac_plain(wc, Y[r][e], C[r][e], lap);
@@ -424,7 +413,7 @@ __device__ inline void fwd_tile_body(const FwdTile<T> &a, const TileView &t, int
                     T out = ac_plain(wc, Y[r][e], C[r][e], lap);
                     if (!pc.X || pc.near(r, e)) {  // uniform for TILE_X
                         const T num = ac_pml_num(k, pc.a2(r, e, k), pc.e(r, e, k), wc, Y[r][e], C[r][e], lap, fs - fn[e],
-                                                 east_of(G[r], e) - west_of(G[r], e));
+                                                 lane_east(G[r][e]) - lane_west(G[r][e]));
                         out = pc.near(r, e) ? pc.div(num, r, e, k) : out;
                     }
                     Y[r][e] = pc.in(r, e) ? out : T(0);
@@ -449,19 +438,19 @@ __device__ inline void fwd_tile_body(const FwdTile<T> &a, const TileView &t, int
             }
         }
         if constexpr (V == 0 && PML) {  // phi/psi from u^n before the sources
-            vst(&lds.v[par][w][0][lv], Y[0]);
-            vst(&lds.v[par][w][1][lv], Y[R - 1]);
+            vst(&lds.v[par][w][0][lane], Y[0]);
+            vst(&lds.v[par][w][1][lane], Y[R - 1]);
             __syncthreads();
             T vn_[VEC], vs_[VEC];
-            vld(vn_, &lds.v[par][wu][1][lv]);
-            vld(vs_, &lds.v[par][wd][0][lv]);
+            vld(vn_, &lds.v[par][wu][1][lane]);
+            vld(vs_, &lds.v[par][wd][0][lane]);
 #pragma unroll
             for (int r = 0; r < R; r++)
 #pragma unroll
                 for (int e = 0; e < VEC; e++) {
                     const T vn = r > 0 ? Y[r > 0 ? r - 1 : r][e] : vn_[e];
                     const T vs = r < R - 1 ? Y[r < R - 1 ? r + 1 : r][e] : vs_[e];
-                    const T ve = east_of(Y[r], e), vw = west_of(Y[r], e);  // (by every lane)
+                    const T ve = lane_east(Y[r][e]), vw = lane_west(Y[r][e]);  // (by every lane)
                     const T ct = C[r][e] * pc.c(r, e);
                     if (ct != T(0)) {
                         F[r][e] = ac_phi(k, pc.d1(r), F[r][e], ct, vs - vn);
@@ -472,7 +461,7 @@ __device__ inline void fwd_tile_body(const FwdTile<T> &a, const TileView &t, int
         // the next level's value is loaded inside the same branch: a load carried to the loop's end
         // on the other path would make every level wait for its own stores
         if (wp.hi > wp.lo) {
-            add_points<T, R, VEC>(a, wp, lrow, lane, lds.plane[w], srow, pv, Y);
+            add_points<T, R>(a, wp, lrow, lane, lds.plane[w], srow, pv, Y);
             srow += ns;
             if (q + 1 < nt) pv = first_point(a.src, wp, lane, srow);
         }
@@ -493,17 +482,17 @@ __device__ inline void fwd_tile_body(const FwdTile<T> &a, const TileView &t, int
     }
 }
 
-// RN (RP): rows per wavefront of a plain (PML) tile; VEC columns per lane.  What bounds it: at 1000^2 x 32
+// RN (RP): rows per wavefront of a plain (PML) tile.  What bounds it: at 1000^2 x 32
 // shots FP32 with 7 levels per launch (63 us per level; one level per launch takes 104) the vector units
 // issue two thirds of the time, half of that for the PML tiles and 40 % for the halo, and 3.3 TB/s move,
 // mostly stores; a workgroup's loads do not overlap its own levels, so several per CU have to.
 // FP32 asks for three (80 VGPRs, a few spilled): 63 us, two 63, four (64 VGPRs) 74.
-template <typename T, int V, int RN, int RP, int VEC, int NW>
+template <typename T, int V, int RN, int RP, int NW>
 __global__ __launch_bounds__(NW *WAVE) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 6 : 4)))
 void ac_fwd_tile(const FwdTile<T> a)
 {
-    using LP = FwdTileLds<T, V, RP, VEC, NW, true>;
-    using LN = FwdTileLds<T, V, RN, VEC, NW, false>;
+    using LP = FwdTileLds<T, V, RP, NW, true>;
+    using LN = FwdTileLds<T, V, RN, NW, false>;
     __shared__ __align__(16) char raw[sizeof(LP) > sizeof(LN) ? sizeof(LP) : sizeof(LN)];
     TileMap m{a.ntiles, a.act, 1, a.nb};
     int z, s, tile;
@@ -512,34 +501,34 @@ void ac_fwd_tile(const FwdTile<T> a)
     const int nt = min(a.nt, a.nstep[s] - a.n + 1);
     LP &lp = *reinterpret_cast<LP *>(raw);
     if (e.w == TILE_PLAIN)
-        fwd_tile_body<T, V, RN, VEC, NW, TILE_PLAIN>(a, tile_view<RN, VEC>(c, e), s, tile, nt,
+        fwd_tile_body<T, V, RN, NW, TILE_PLAIN>(a, tile_view<RN>(c, e), s, tile, nt,
                                                      *reinterpret_cast<LN *>(raw));
     else if (e.w == TILE_X)
-        fwd_tile_body<T, V, RP, VEC, NW, TILE_X>(a, tile_view<RP, VEC>(c, e), s, tile, nt, lp);
+        fwd_tile_body<T, V, RP, NW, TILE_X>(a, tile_view<RP>(c, e), s, tile, nt, lp);
     else if (e.w == TILE_Y)
-        fwd_tile_body<T, V, RP, VEC, NW, TILE_Y>(a, tile_view<RP, VEC>(c, e), s, tile, nt, lp);
+        fwd_tile_body<T, V, RP, NW, TILE_Y>(a, tile_view<RP>(c, e), s, tile, nt, lp);
     else
-        fwd_tile_body<T, V, RP, VEC, NW, TILE_XY>(a, tile_view<RP, VEC>(c, e), s, tile, nt, lp);
+        fwd_tile_body<T, V, RP, NW, TILE_XY>(a, tile_view<RP>(c, e), s, tile, nt, lp);
 }
 
 // ---------------------------------------------------------------------------------------------
 // adjoint
 // ---------------------------------------------------------------------------------------------
-template <typename T, int V, int R, int VEC, int NW, bool PML> struct AdjTileLds {
-    T p[2][NW][2][WAVE * VEC];
-    T f[PML ? 2 : 0][NW][2][WAVE * VEC];  // C (tau - sigma) F rows
-    T plane[NW][R + (PML ? 2 : 0)][WAVE * VEC];
+template <typename T, int V, int R, int NW, bool PML> struct AdjTileLds {
+    T p[2][NW][2][WAVE];
+    T f[PML ? 2 : 0][NW][2][WAVE];  // C (tau - sigma) F rows
+    T plane[NW][R + (PML ? 2 : 0)][WAVE];
 };
 
-template <typename T, int V, int R, int VEC, int NW, int KIND, bool DENSE>
+template <typename T, int V, int R, int NW, int KIND, bool DENSE>
 __device__ inline void adj_tile_body(const AdjTile<T> &a, const TileView &t, int g, int tile,
-                                     AdjTileLds<T, V, R, VEC, NW, KIND != TILE_PLAIN> &lds)
+                                     AdjTileLds<T, V, R, NW, KIND != TILE_PLAIN> &lds)
 {
     constexpr bool PML = KIND != TILE_PLAIN;
     constexpr bool UN = V == 0 && PML;  // kernel 0 also reads u^n before its sources
     constexpr int RD = DENSE ? R : 1, RV = UN ? R + 2 : 1;
     const AcCoef<T> k = a.k;
-    const int lane = t.lane, w = t.w, j = t.j, lv = lane * VEC;
+    const int lane = t.lane, w = t.w, j = t.j;
     const uint32_t jb = (uint32_t)j * (uint32_t)sizeof(T), jcb = (uint32_t)t.jc * (uint32_t)sizeof(T);
     const int lrow = w * R;
     const int m = a.n - a.nt + 1;
@@ -547,9 +536,9 @@ __device__ inline void adj_tile_body(const AdjTile<T> &a, const TileView &t, int
     const int wu = max(w - 1, 0), wd = min(w + 1, NW - 1);
     const T zero[VEC] = {};
 #pragma unroll
-    for (int r = 0; r < R + (PML ? 2 : 0); r++) vst(&lds.plane[w][r][lv], zero);
+    for (int r = 0; r < R + (PML ? 2 : 0); r++) vst(&lds.plane[w][r][lane], zero);
 
-    PmlCoef<T, R, VEC, KIND> pc;
+    PmlCoef<T, R, KIND> pc;
     if constexpr (PML) pc.load(t, a, k);
     uint32_t ro[R + 2];  // byte offset of rows r0 - 1 .. r0 + R, clamped to the extent and the grid
 #pragma unroll
@@ -625,8 +614,8 @@ __device__ inline void adj_tile_body(const AdjTile<T> &a, const TileView &t, int
                     for (int q = 0; q < R + 2; q++) recompute(C[q][e]);
                 }
             }
-            vst(&lds.p[par][w][0][lv], X[0]);
-            vst(&lds.p[par][w][1][lv], X[R - 1]);
+            vst(&lds.p[par][w][0][lane], X[0]);
+            vst(&lds.p[par][w][1][lane], X[R - 1]);
             // (C (tau - sigma)) F of a row
             auto fq = [&](int r, T (&o)[VEC]) {
 #pragma unroll
@@ -646,8 +635,8 @@ __device__ inline void adj_tile_body(const AdjTile<T> &a, const TileView &t, int
                 T q0[VEC], q1[VEC];
                 fq(0, q0);
                 fq(R - 1, q1);
-                vst(&lds.f[par][w][0][lv], q0);
-                vst(&lds.f[par][w][1][lv], q1);
+                vst(&lds.f[par][w][0][lane], q0);
+                vst(&lds.f[par][w][1][lane], q1);
             }
             // the next level's inputs, in flight during this one
             if (n > m) {
@@ -656,8 +645,8 @@ __device__ inline void adj_tile_body(const AdjTile<T> &a, const TileView &t, int
             }
             __syncthreads();
             T pn_[VEC], ps_[VEC];
-            vld(pn_, &lds.p[par][wu][1][lv]);
-            vld(ps_, &lds.p[par][wd][0][lv]);
+            vld(pn_, &lds.p[par][wu][1][lane]);
+            vld(ps_, &lds.p[par][wd][0][lane]);
             if constexpr (UN) {  // F^n, G^n and their dL/dC terms, with u^n before its sources
                 if (wsrc.hi > wsrc.lo) {
                     sum_points(a.src, wsrc, lrow - 1, lane, lds.plane[w], srow,
@@ -666,8 +655,8 @@ __device__ inline void adj_tile_body(const AdjTile<T> &a, const TileView &t, int
                     for (int q = 0; q < RV; q++)
                         if (wsrc.rows >> q & 1) {
 #pragma unroll
-                            for (int e = 0; e < VEC; e++) VN[q][e] -= lds.plane[w][q][lv + e];
-                            vst(&lds.plane[w][q][lv], zero);
+                            for (int e = 0; e < VEC; e++) VN[q][e] -= lds.plane[w][q][lane];
+                            vst(&lds.plane[w][q][lane], zero);
                         }
                     __builtin_amdgcn_wave_barrier();
                     srow -= ns;
@@ -678,21 +667,21 @@ __device__ inline void adj_tile_body(const AdjTile<T> &a, const TileView &t, int
                     for (int e = 0; e < VEC; e++) {
                         const T pn = r > 0 ? X[r > 0 ? r - 1 : r][e] : pn_[e];
                         const T ps = r < R - 1 ? X[r < R - 1 ? r + 1 : r][e] : ps_[e];
-                        const T dp = west_of(X[r], e) - east_of(X[r], e);
-                        const T dvj = east_of(VN[UN ? r + 1 : 0], e) - west_of(VN[UN ? r + 1 : 0], e);
+                        const T dp = lane_west(X[r][e]) - lane_east(X[r][e]);
+                        const T dvj = lane_east(VN[UN ? r + 1 : 0][e]) - lane_west(VN[UN ? r + 1 : 0][e]);
                         adj_phipsi(r, e, pn - ps, dp, VN[UN ? r + 2 : 0][e] - VN[UN ? r : 0][e], dvj, F[r][e], G[r][e], acc[r][e]);
                     }
                 T q0[VEC], q1[VEC];
                 fq(0, q0);
                 fq(R - 1, q1);
-                vst(&lds.f[par][w][0][lv], q0);
-                vst(&lds.f[par][w][1][lv], q1);
+                vst(&lds.f[par][w][0][lane], q0);
+                vst(&lds.f[par][w][1][lane], q1);
                 __syncthreads();
             }
             T fn[VEC], fs_[VEC], fc[VEC], fs[VEC];
             if constexpr (PML) {
-                vld(fn, &lds.f[par][wu][1][lv]);
-                vld(fs_, &lds.f[par][wd][0][lv]);
+                vld(fn, &lds.f[par][wu][1][lane]);
+                vld(fs_, &lds.f[par][wd][0][lane]);
                 fq(0, fc);
             }
             if (wr.hi > wr.lo) sum_points(a.rcv, wr, lrow, lane, lds.plane[w], rrow, rv, T(1));
@@ -720,13 +709,13 @@ __device__ inline void adj_tile_body(const AdjTile<T> &a, const TileView &t, int
 #pragma unroll
                 for (int e = 0; e < VEC; e++) {
                     const T p1c = X[r][e];
-                    const T lapq = ac_lap(k, qc[e], qs[e], qn[e], east_of(qc, e), west_of(qc, e));
+                    const T lapq = ac_lap(k, qc[e], qs[e], qn[e], lane_east(qc[e]), lane_west(qc[e]));
                     T Pv = ac_fma(T(2), p1c, lapq) - Y[r][e];
                     if constexpr (DENSE) Pv += D[r][e];
                     if constexpr (PML) {
                         if (!pc.X || pc.near(r, e)) {  // uniform for TILE_X
                             T U_ = pc.a2(r, e, k) * p1c + lapq - pc.e(r, e, k) * Y[r][e] + k.fx * (fn[e] - fs[e]) +
-                                   k.fy * (west_of(gq, e) - east_of(gq, e));
+                                   k.fy * (lane_west(gq[e]) - lane_east(gq[e]));
                             if constexpr (DENSE) U_ += D[r][e];
                             Pv = pc.near(r, e) ? pc.div(U_, r, e, k) : Pv;
                         }
@@ -737,24 +726,24 @@ __device__ inline void adj_tile_body(const AdjTile<T> &a, const TileView &t, int
                 if (wr.rows >> r & 1) {  // uniform: receiver residuals on this row
 #pragma unroll
                     for (int e = 0; e < VEC; e++) {
-                        const T add = lds.plane[w][r][lv + e];
+                        const T add = lds.plane[w][r][lane];
                         if constexpr (PML) Y[r][e] += pc.div(add, r, e, k);
                         else Y[r][e] += add;
                     }
-                    vst(&lds.plane[w][r][lv], zero);
+                    vst(&lds.plane[w][r][lane], zero);
                 }
 #pragma unroll
                 for (int e = 0; e < VEC; e++)
                     acc[r][e] = ac_fma(Y[r][e],
-                                       ac_lap(k, U[r + 1][e], U[r + 2][e], U[r][e], east_of(U[r + 1], e), west_of(U[r + 1], e)),
+                                       ac_lap(k, U[r + 1][e], U[r + 2][e], U[r][e], lane_east(U[r + 1][e]), lane_west(U[r + 1][e])),
                                        acc[r][e]);
                 if constexpr (PML && V == 1) {
 #pragma unroll
                     for (int e = 0; e < VEC; e++) {
                         const T pn = r > 0 ? X[r > 0 ? r - 1 : r][e] : pn_[e];
                         const T ps = r < R - 1 ? X[r < R - 1 ? r + 1 : r][e] : ps_[e];
-                        adj_phipsi(r, e, pn - ps, west_of(X[r], e) - east_of(X[r], e), U[r + 2][e] - U[r][e],
-                                   east_of(U[r + 1], e) - west_of(U[r + 1], e), F[r][e], G[r][e], acc[r][e]);
+                        adj_phipsi(r, e, pn - ps, lane_west(X[r][e]) - lane_east(X[r][e]), U[r + 2][e] - U[r][e],
+                                   lane_east(U[r + 1][e]) - lane_west(U[r + 1][e]), F[r][e], G[r][e], acc[r][e]);
                     }
                 }
 #pragma unroll
@@ -809,19 +798,19 @@ __device__ inline void adj_tile_body(const AdjTile<T> &a, const TileView &t, int
         T *p = at_off(at_off(gC, ro[r + 1]), jb);
 #pragma unroll
         for (int e = 0; e < VEC; e++)
-            if (j + e >= t.j0 && j + e < t.j1 && (!PML || pc.in(r, e))) p[e] += acc[r][e];
+            if (j >= t.j0 && j < t.j1 && (!PML || pc.in(r, e))) p[e] += acc[r][e];
     }
 }
 
 // Bounds as in the forward; 1000^2 x 32 shots FP32, 7 levels per launch: 94 us per level (one level per
 // launch and a receiver launch: 178).  Two workgroups per CU in FP32 (128 VGPRs with a few spilled): 100
 // against 147 us with one (no spills) and 203 with three, eight shots per workgroup.
-template <typename T, int V, int RN, int RP, int VEC, int NW, bool DENSE>
+template <typename T, int V, int RN, int RP, int NW, bool DENSE>
 __global__ __launch_bounds__(NW *WAVE) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 4 : 2)))
 void ac_adj_tile(const AdjTile<T> a)
 {
-    using LP = AdjTileLds<T, V, RP, VEC, NW, true>;
-    using LN = AdjTileLds<T, V, RN, VEC, NW, false>;
+    using LP = AdjTileLds<T, V, RP, NW, true>;
+    using LN = AdjTileLds<T, V, RN, NW, false>;
     __shared__ __align__(16) char raw[sizeof(LP) > sizeof(LN) ? sizeof(LP) : sizeof(LN)];
     TileMap m{a.ntiles, (a.act + a.Sg - 1) / a.Sg, 1, a.nb};
     int z, g, tile;
@@ -829,14 +818,14 @@ void ac_adj_tile(const AdjTile<T> a)
     const int4 c = a.tiles[2 * tile], e = a.tiles[2 * tile + 1];
     LP &lp = *reinterpret_cast<LP *>(raw);
     if (e.w == TILE_PLAIN)
-        adj_tile_body<T, V, RN, VEC, NW, TILE_PLAIN, DENSE>(a, tile_view<RN, VEC>(c, e), g, tile,
+        adj_tile_body<T, V, RN, NW, TILE_PLAIN, DENSE>(a, tile_view<RN>(c, e), g, tile,
                                                             *reinterpret_cast<LN *>(raw));
     else if (e.w == TILE_X)
-        adj_tile_body<T, V, RP, VEC, NW, TILE_X, DENSE>(a, tile_view<RP, VEC>(c, e), g, tile, lp);
+        adj_tile_body<T, V, RP, NW, TILE_X, DENSE>(a, tile_view<RP>(c, e), g, tile, lp);
     else if (e.w == TILE_Y)
-        adj_tile_body<T, V, RP, VEC, NW, TILE_Y, DENSE>(a, tile_view<RP, VEC>(c, e), g, tile, lp);
+        adj_tile_body<T, V, RP, NW, TILE_Y, DENSE>(a, tile_view<RP>(c, e), g, tile, lp);
     else
-        adj_tile_body<T, V, RP, VEC, NW, TILE_XY, DENSE>(a, tile_view<RP, VEC>(c, e), g, tile, lp);
+        adj_tile_body<T, V, RP, NW, TILE_XY, DENSE>(a, tile_view<RP>(c, e), g, tile, lp);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -849,14 +838,14 @@ struct TileHost {
 // Tiles covering rows [ilo, ihi) x columns [jlo, jhi) with halo H; sx, ty: the damping profiles of the
 // padded axes (as the kernels read them).
 struct TileGrid {
-    int NX, NY, rowsN, rowsP, vec;  // interior cells; rows of a plain / PML tile; columns per lane
+    int NX, NY, rowsN, rowsP;  // interior cells; rows of a plain / PML tile
     std::vector<int> px, py;        // prefix counts of the rows (columns) in the PML or next to it
     std::vector<int> rx, ry;        // of those on the ring
 };
 template <typename T>
-static inline TileGrid tile_grid(const std::vector<T> &sx, const std::vector<T> &ty, int rowsN, int rowsP, int vec)
+static inline TileGrid tile_grid(const std::vector<T> &sx, const std::vector<T> &ty, int rowsN, int rowsP)
 {
-    TileGrid g{(int)sx.size() - 2, (int)ty.size() - 2, rowsN, rowsP, vec, {0}, {0}, {0}, {0}};
+    TileGrid g{(int)sx.size() - 2, (int)ty.size() - 2, rowsN, rowsP, {0}, {0}, {0}, {0}};
     auto count = [](const std::vector<T> &f, std::vector<int> &near, std::vector<int> &ring) {
         for (size_t q = 0; q < f.size(); q++) {
             const bool n = f[q] != T(0) || (q > 0 && f[q - 1] != T(0)) || (q + 1 < f.size() && f[q + 1] != T(0));
@@ -882,13 +871,13 @@ static inline void add_tiles(std::vector<TileHost> &out, const TileGrid &g, int 
                              bool plain)
 {
     if (ihi <= ilo || jhi <= jlo) return;
-    const std::vector<int> ci = tile_cuts(ilo, ihi, H, g.NX + 2, plain ? g.rowsN : g.rowsP, 1);
-    const std::vector<int> cj = tile_cuts(jlo, jhi, H, g.NY + 2, WAVE * g.vec, g.vec);
+    const std::vector<int> ci = tile_cuts(ilo, ihi, H, g.NX + 2, plain ? g.rowsN : g.rowsP);
+    const std::vector<int> cj = tile_cuts(jlo, jhi, H, g.NY + 2, WAVE);
     for (size_t p = 0; p + 1 < ci.size(); p++)
         for (size_t q = 0; q + 1 < cj.size(); q++) {
             TileHost t{ci[p], ci[p + 1], cj[q], cj[q + 1], 0, 0, 0, 0, 0};
             t.ie = std::max(t.i0 - H, 0);
-            t.je = std::max(t.j0 - H, 0) / g.vec * g.vec;
+            t.je = std::max(t.j0 - H, 0);
             t.ne = std::min(t.i1 + H, g.NX + 2) - t.ie;
             t.ce = std::min(t.j1 + H, g.NY + 2) - t.je;
             t.kind = tile_kind(g, t);
@@ -904,10 +893,9 @@ static inline void add_tiles(std::vector<TileHost> &out, const TileGrid &g, int 
 static inline std::vector<TileHost> make_tiles(int variant, int levels, const Rect &R, const TileGrid &g)
 {
     std::vector<TileHost> a, b;
-    const int H = variant == 0 ? 2 * levels : levels, X = g.NX + 2, Y = g.NY + 2, v = g.vec;
+    const int H = variant == 0 ? 2 * levels : levels, X = g.NX + 2, Y = g.NY + 2;
     add_tiles(a, g, 0, X, 0, Y, H, false);
-    // the bands' and the plain tiles' columns meet at multiples of vec
-    const Rect Q{R.iL + levels, R.iR - levels, (R.jL + levels + v - 1) / v * v, (R.jR - levels) / v * v};
+    const Rect Q{R.iL + levels, R.iR - levels, R.jL + levels, R.jR - levels};
     if (Q.iR <= Q.iL || Q.jR <= Q.jL) return a;
     add_tiles(b, g, Q.iL, Q.iR, Q.jL, Q.jR, levels, true);
     for (const TileHost &t : b)

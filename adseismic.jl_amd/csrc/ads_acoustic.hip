@@ -725,8 +725,8 @@ template <typename T> struct AcPlan : AcPlanBase {
         double levels = 0.0;
         for (int q = 0; q < a.nt; q++) levels += active[a.n + q];
         int pr = prof_start(ADS_PROF_AC_FWD, st);
-        if (variant == 1) ac_fwd_tile<T, 1, TILE_RN, TILE_RP, 1, TILE_WAVES><<<nb, TILE_WAVES * WAVE, 0, st>>>(a);
-        else ac_fwd_tile<T, 0, TILE_RN, TILE_RP, 1, TILE_WAVES><<<nb, TILE_WAVES * WAVE, 0, st>>>(a);
+        if (variant == 1) ac_fwd_tile<T, 1, TILE_RN, TILE_RP, TILE_WAVES><<<nb, TILE_WAVES * WAVE, 0, st>>>(a);
+        else ac_fwd_tile<T, 0, TILE_RN, TILE_RP, TILE_WAVES><<<nb, TILE_WAVES * WAVE, 0, st>>>(a);
         // per launch: u^{n-1}, u^{n-2}, C and phi/psi once, phi/psi back once, every level's u
         prof_stop(pr, st, cell_bytes() * (levels + a.act * (3.0 + 4.0 * f_pml)), a.nt);
         ADS_LAUNCH_CHECK();
@@ -742,8 +742,8 @@ template <typename T> struct AcPlan : AcPlanBase {
         double levels = 0.0;
         for (int q = 0; q < a.nt; q++) levels += active[a.n - q];
         int pr = prof_start(ADS_PROF_AC_ADJ, st);
-        if (variant == 1) ac_adj_tile<T, 1, TILE_RN, TILE_RP, 1, TILE_WAVES, DENSE><<<nb, TILE_WAVES * WAVE, 0, st>>>(a);
-        else ac_adj_tile<T, 0, TILE_RN, TILE_RP, 1, TILE_WAVES, DENSE><<<nb, TILE_WAVES * WAVE, 0, st>>>(a);
+        if (variant == 1) ac_adj_tile<T, 1, TILE_RN, TILE_RP, TILE_WAVES, DENSE><<<nb, TILE_WAVES * WAVE, 0, st>>>(a);
+        else ac_adj_tile<T, 0, TILE_RN, TILE_RP, TILE_WAVES, DENSE><<<nb, TILE_WAVES * WAVE, 0, st>>>(a);
         // per launch: P^{n+1}, P^{n+2} and F/G in and out, C and dL/dC in and out once per group of shots, and
         // every level's u (kernel 0's PML: one more) and dense cotangent
         const double per_shot = 4.0 + (variant == 1 ? 4.0 : 5.0) * f_pml;
@@ -1170,7 +1170,7 @@ static int build_tiles(AcPlan<T> *P, const Rect &R, const std::vector<int64_t> &
 {
     const int NX = (int)P->NX, NY = (int)P->NY;
     const std::vector<T> sx(P->sx.begin(), P->sx.end()), ty(P->ty.begin(), P->ty.end());
-    const TileGrid grid = tile_grid(sx, ty, TILE_WAVES * TILE_RN, TILE_WAVES * TILE_RP, 1);
+    const TileGrid grid = tile_grid(sx, ty, TILE_WAVES * TILE_RN, TILE_WAVES * TILE_RP);
     P->tile_levels = choose_levels(P->variant, P->nshots, sizeof(T), R, grid);
     const std::vector<TileHost> tiles = make_tiles(P->variant, P->tile_levels, R, grid);
     std::vector<int4> t;

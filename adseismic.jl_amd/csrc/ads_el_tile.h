@@ -410,7 +410,7 @@ static inline std::vector<ElTileHost> el_tiles(int NX, int NY, int levels, int r
 {
     std::vector<ElTileHost> out;
     const int H = 4 * levels;
-    const std::vector<int> ci = tile_cuts(0, NX + 2, H, NX + 2, rows, 1), cj = tile_cuts(0, NY + 2, H, NY + 2, WAVE, 1);
+    const std::vector<int> ci = tile_cuts(0, NX + 2, H, NX + 2, rows), cj = tile_cuts(0, NY + 2, H, NY + 2, WAVE);
     for (size_t p = 0; p + 1 < ci.size(); p++)
         for (size_t q = 0; q + 1 < cj.size(); q++) {
             ElTileHost t{ci[p], ci[p + 1], cj[q], cj[q + 1], 0, 0, 0, 0, 0};

@@ -45,21 +45,20 @@ template <int R> __device__ inline uint32_t row_mask(int r0, int lo, int hi)
     return __builtin_amdgcn_readfirstlane((1u << b) - (1u << min(a, b)));
 }
 
-// Cuts [lo, hi) into equal pieces whose extents (halo H, clipped to [0, n), starting at a multiple
-// of unit) fit in cap cells.
-static inline std::vector<int> tile_cuts(int lo, int hi, int H, int n, int cap, int unit)
+// Cuts [lo, hi) into equal pieces whose extents (halo H, clipped to [0, n)) fit in cap cells.
+static inline std::vector<int> tile_cuts(int lo, int hi, int H, int n, int cap)
 {
     // pieces away from the grid's edges hold at most cap - 2 H cells, the two at its edges H more
-    const int len = hi - lo, in = std::max(cap - 2 * H, unit);
+    const int len = hi - lo, in = std::max(cap - 2 * H, 1);
     for (int k = std::max(1, (len - 2 * H) / in);; k++) {
         std::vector<int> c;
-        const int size = ((len + k - 1) / k + unit - 1) / unit * unit;
+        const int size = (len + k - 1) / k;
         for (int x = lo; x < hi; x += size) c.push_back(x);
         c.push_back(hi);
         bool ok = true;
         for (size_t q = 0; q + 1 < c.size(); q++)
-            ok = ok && std::min(c[q + 1] + H, n) - std::max(c[q] - H, 0) / unit * unit <= cap;
-        if (ok || size <= unit) return c;
+            ok = ok && std::min(c[q + 1] + H, n) - std::max(c[q] - H, 0) <= cap;
+        if (ok || size <= 1) return c;
     }
 }
 
