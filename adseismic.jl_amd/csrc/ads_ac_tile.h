@@ -486,7 +486,7 @@ __device__ inline void fwd_tile_body(const FwdTile<T> &a, const TileView &t, int
 // shots FP32 with 7 levels per launch (63 us per level; one level per launch takes 104) the vector units
 // issue two thirds of the time, half of that for the PML tiles and 40 % for the halo, and 3.3 TB/s move,
 // mostly stores; a workgroup's loads do not overlap its own levels, so several per CU have to.
-// FP32 asks for three (80 VGPRs, a few spilled): 63 us, two 63, four (64 VGPRs) 74.
+// FP32 asks for three (69 VGPRs): 63 us, two 63, four (64 VGPRs, some spilled) 74.
 template <typename T, int V, int RN, int RP, int NW>
 __global__ __launch_bounds__(NW *WAVE) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 6 : 4)))
 void ac_fwd_tile(const FwdTile<T> a)

@@ -314,16 +314,19 @@ int ads_acoustic_plan_set_shape(ads_acoustic_plan *plan, const int *shape);
 /* hipGraph replay (no counterpart in the reference): with enable = 1, each checkpoint segment
  * of the forward sweep, of the recomputation and of the adjoint sweep is captured once into a
  * graph (on a private stream) and replayed on the caller's stream afterwards.  A graph is keyed
- * by the segment, the workspace, srcv, traces and residual addresses; calls with other buffers
- * capture new graphs.  Graphs are not used while ads_profile_begin() timing is active, and are
- * dropped by set_shape/autotune and at plan destruction. */
+ * by the segment, the workspace (its address and layout), srcv, traces and residual addresses;
+ * calls with other buffers capture new graphs.  Graphs are not used while ads_profile_begin()
+ * timing is active, and are dropped by set_shape/autotune and at plan destruction.  With graphs
+ * off, several threads may run one plan at a time, each with a workspace and outputs of its own;
+ * with graphs on, and for the calls that set something, a plan belongs to one thread. */
 int ads_acoustic_plan_set_graph(ads_acoustic_plan *plan, int enable);
 
 /* Temporal blocking of the forward sweeps (no counterpart in the reference): with levels = 2 (the default)
- * a launch advances several time levels (seven with PropagatorKernel 1 or 2, four with 0), each
- * workgroup holding one tile of the grid with a halo in registers; with levels = 1 every level is a launch
- * of its own.  Results are bit-identical.  ads_acoustic_plan_blocking returns 2 when levels = 2 is set and
- * no source lies in the interior rectangle (the cells that no PML term reaches), else 1. */
+ * a launch advances several time levels (a number that the plan chooses from its grid and shots: 7 to 12
+ * with PropagatorKernel 1 or 2, 3 to 7 with 0), each workgroup holding one tile of the grid with a halo in
+ * registers; with levels = 1 every level is a launch of its own.  Results are bit-identical.  Sources may lie
+ * anywhere.  ads_acoustic_plan_blocking tells, as it did before the tiles took such sources, whether levels = 2
+ * is set and no source lies in the interior rectangle (the cells that no PML term reaches): 2 if so, else 1. */
 int ads_acoustic_plan_set_blocking(ads_acoustic_plan *plan, int levels);
 int ads_acoustic_plan_blocking(const ads_acoustic_plan *plan);
 
@@ -331,8 +334,9 @@ int ads_acoustic_plan_blocking(const ads_acoustic_plan *plan);
 int ads_acoustic_plan_set_frame_rows(ads_acoustic_plan *plan, int rows);
 
 /* Plain drop-in of AcousticPropagatorSolver (Core.jl:562-620) on the plan's shots (every shot
- * must have nstep == NSTEP): writes the full histories u, phi, psi, each laid out
- * [shot][level 0..NSTEP][N] (phi/psi may be NULL).  scratch: device buffer of
+ * must have nstep == NSTEP, ADS_ERR_SHAPE otherwise): writes the full histories u, phi, psi, each
+ * laid out [shot][level 0..NSTEP][N] (either or both of phi and psi may be NULL; one alone is
+ * slower, a level per launch and a copy).  scratch: device buffer of
  * ads_acoustic_plan_history_scratch_size() bytes. */
 size_t ads_acoustic_plan_history_scratch_size(const ads_acoustic_plan *plan);
 int ads_acoustic_plan_forward_history(ads_acoustic_plan *plan, const void *model,
@@ -404,7 +408,7 @@ int ads_elastic_plan_backward_dense(ads_elastic_plan *plan, const void *rho, con
                                     void *grad_rho, void *grad_lam, void *grad_mu, void *workspace,
                                     size_t ws_bytes, int64_t K, ads_stream_t stream);
 /* Plain drop-in of ElasticPropagatorSolver (Core.jl:31-94): the full histories of every shot
- * (nstep == NSTEP), dense layout [shot][field vx, vy, sxx, syy, sxy][level 0..NSTEP][N].
+ * (nstep == NSTEP, ADS_ERR_SHAPE otherwise), dense layout [shot][field vx, vy, sxx, syy, sxy][level 0..NSTEP][N].
  * scratch: ads_elastic_plan_history_scratch_size() bytes (CPML memory variables). */
 size_t ads_elastic_plan_history_scratch_size(const ads_elastic_plan *plan);
 int ads_elastic_forward_history(ads_elastic_plan *plan, const void *rho, const void *lam,
