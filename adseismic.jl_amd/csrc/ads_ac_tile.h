@@ -626,10 +626,17 @@ __device__ inline void adj_tile_body(const AdjTile<T> &a, const TileView &t, int
             auto adj_phipsi = [&](int r, int e, T dpi, T dpj, T dvi, T dvj, T &F, T &G, T &acc) {
                 const T c = pc.c(r, e);
                 const bool pml = pc.in(r, e) && pc.pml(r, e);
-                F = pml ? pc.d1(r) * F + k.ex * dpi : T(0);
-                G = pml ? pc.tk[e] * G + k.ey * dpj : T(0);
-                acc = ac_fma(F * c * k.fx, dvi, acc);
-                acc = ac_fma(G * -c * k.fy, dvj, acc);
+                if constexpr (V == 1) {  // (a dv that is not finite makes the cell's other term so, too)
+                    F = pml ? pc.d1(r) * F + k.ex * dpi : T(0);
+                    G = pml ? pc.tk[e] * G + k.ey * dpj : T(0);
+                    acc = ac_fma(F * c * k.fx, dvi, acc);
+                    acc = ac_fma(G * -c * k.fy, dvj, acc);
+                } else if (pml) {  // elsewhere F and G stay 0, and nothing joins acc beside any dv
+                    F = pc.d1(r) * F + k.ex * dpi;
+                    G = pc.tk[e] * G + k.ey * dpj;
+                    acc = ac_fma(F * c * k.fx, dvi, acc);
+                    acc = ac_fma(G * -c * k.fy, dvj, acc);
+                }
             };
             if constexpr (PML && V == 1) {
                 T q0[VEC], q1[VEC];

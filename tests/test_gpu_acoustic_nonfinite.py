@@ -41,3 +41,24 @@ def test_infinite_source(ads, cuda, kernel, dtype, NX, NY, si, sj, hy):
     out = torch.as_tensor(~pml, device="cuda")
     out[0] = out[-1] = out[:, 0] = out[:, -1] = True
     assert (phi[0][:, out] == 0).all() and (psi[0][:, out] == 0).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("kernel", [0, 1])
+def test_infinite_last_sample(ads, cuda, kernel, dtype):
+    """The last level's source sample reaches the source cell of the last level alone, which no receiver there reads and
+    no dL/dC term uses unless the cell touches the PML: an infinite one leaves the gradient as it is."""
+    p = ads.AcousticPropagatorParams(NX=30, NY=62, NSTEP=40, DELTAX=10.0, DELTAY=10.0, DELTAT=1e-3, NPOINTS_PML=8,
+                                     vp_ref=2000.0, PropagatorKernel=kernel)
+    c = torch.linspace(1800.0, 2300.0, 32 * 64, dtype=dtype, device="cuda").reshape(32, 64)
+    out = []
+    for last in (0.0, np.inf):
+        w = 1e3 * np.sin(0.4 * np.arange(40))
+        w[-1] = last
+        plan = ads.AcousticPlan(p, [ads.AcousticSource([16], [30], w[:, None])],
+                                [ads.AcousticReceiver(np.arange(2, 32), np.full(30, 12))], dtype=dtype)
+        srcv = plan.pack_srcv([w[:, None]])
+        obs = torch.ones(plan.trace_elems, dtype=dtype, device="cuda")
+        out.append(plan.gradient(c, srcv, obs, 9)[1].clone())
+    assert torch.isfinite(out[0]).all() and float(out[0].abs().max()) > 0.0
+    assert torch.equal(out[1], out[0])
