@@ -102,9 +102,10 @@ __device__ inline T ac_pml_num(const AcCoef<T> &k, T a2, T e, T wc, T wold, T C,
     return a2 * wc + C * lap + k.ex * dphi + k.ey * dpsi - e * wold;
 }
 // phi^n = (1 - dt sigma) phi + C (tau - sigma) fx dv, psi^n = (1 - dt tau) psi - C (tau - sigma) fy dv;
-// d1 the damping factor, ct = C (tau - sigma).  Taken where ct != 0 only: elsewhere phi and psi stay the 0 that
-// they start from, also beside a dv that is not finite.  (In the tiles the comparison costs no register
-// over the levels and no time; the flags "interior" and "in the PML" cost up to 2.6 %.)
+// d1 the damping factor, ct = C (tau - sigma).  Taken on the interior's PML cells only: elsewhere phi and psi stay
+// the 0 that they start from, also beside a dv that is not finite.  (The tiles tell those cells by
+// C (tau + sigma) != 0, with C = 0 outside the interior, which costs no register over the levels and no time;
+// flags of the cell cost up to 2.6 %.)
 template <typename T> __device__ inline T ac_phi(const AcCoef<T> &k, T d1, T phi, T ct, T dv)
 {
     return d1 * phi + ct * k.fx * dv;
@@ -207,6 +208,8 @@ template <typename T, int R, int KIND> struct PmlCoef {
     }
     // inside the PML
     __device__ inline bool pml(int r, int e) const { return (!X && tu[e] != T(0)) || (!Y && sg[r] != T(0)); }
+    // tau + sigma
+    __device__ inline T sum(int r, int e) const { return X ? sg[r] : Y ? tu[e] : sg[r] + tu[e]; }
     // tau - sigma
     __device__ inline T c(int r, int e) const { return X ? -sg[r] : Y ? tu[e] : tu[e] - sg[r]; }
     __device__ inline T a2(int r, int e, const AcCoef<T> &k) const { return XY ? T(2) - sg[r] * tu[e] * k.dt2 : T(2); }
@@ -421,7 +424,7 @@ __device__ inline void fwd_tile_body(const FwdTile<T> &a, const TileView &t, int
                         const T ct = C[r][e] * pc.c(r, e);
                         F_[e] = F[r][e];
                         G_[e] = G[r][e];
-                        if (ct != T(0)) {
+                        if (C[r][e] * pc.sum(r, e) != T(0)) {
                             F_[e] = ac_phi(k, pc.d1(r), F[r][e], ct, ws - wn);
                             G_[e] = ac_psi(k, pc.tk[e], G[r][e], ct, we - ww);
                         }
@@ -452,7 +455,7 @@ __device__ inline void fwd_tile_body(const FwdTile<T> &a, const TileView &t, int
                     const T vs = r < R - 1 ? Y[r < R - 1 ? r + 1 : r][e] : vs_[e];
                     const T ve = lane_east(Y[r][e]), vw = lane_west(Y[r][e]);  // (by every lane)
                     const T ct = C[r][e] * pc.c(r, e);
-                    if (ct != T(0)) {
+                    if (C[r][e] * pc.sum(r, e) != T(0)) {
                         F[r][e] = ac_phi(k, pc.d1(r), F[r][e], ct, vs - vn);
                         G[r][e] = ac_psi(k, pc.tk[e], G[r][e], ct, ve - vw);
                     }

@@ -238,9 +238,9 @@ __device__ inline void fwd_frame_body(const FwdArgs<T> &a, const TileMap &map,
             const T out = in ? (near ? ac_div(num, den, T(1) / den) : plain) : T(0);
             if (act) u[row + j] = out;
             if (V == 1 && lp) {
-                const T ct = in ? Cij * (tu - s_) : T(0);
-                a.phio.at(s)[row + j] = ct != T(0) ? ac_phi(k, T(1) - k.dt * s_, PH[r + 1], ct, ws - wn) : T(0);
-                a.psio.at(s)[row + j] = ct != T(0) ? ac_psi(k, T(1) - k.dt * tu, PS[r], ct, we - ww) : T(0);
+                const bool pml = in && (s_ != T(0) || tu != T(0));
+                a.phio.at(s)[row + j] = pml ? ac_phi(k, T(1) - k.dt * s_, PH[r + 1], Cij * (tu - s_), ws - wn) : T(0);
+                a.psio.at(s)[row + j] = pml ? ac_psi(k, T(1) - k.dt * tu, PS[r], Cij * (tu - s_), we - ww) : T(0);
             }
         }
     }
@@ -265,10 +265,9 @@ __global__ __launch_bounds__(256) void ac_fwd_phipsi(
         const int i = m.x + r;
         if (i < 1 || i > NX || !(pmlx[i] | pmly[j])) continue;
         const int64_t ij = (int64_t)i * P + j;
-        const T sg = sx[i], ct = C[ij] * (tu - sg);
-        if (ct == T(0)) continue;  // both buffers hold 0 there
-        phio.at(s)[ij] = ac_phi(k, T(1) - k.dt * sg, phi_.at(s)[ij], ct, u[ij + P] - u[ij - P]);
-        psio.at(s)[ij] = ac_psi(k, T(1) - k.dt * tu, psi_.at(s)[ij], ct, u[ij + 1] - u[ij - 1]);
+        const T sg = sx[i], Cij = C[ij];
+        phio.at(s)[ij] = ac_phi(k, T(1) - k.dt * sg, phi_.at(s)[ij], Cij * (tu - sg), u[ij + P] - u[ij - P]);
+        psio.at(s)[ij] = ac_psi(k, T(1) - k.dt * tu, psi_.at(s)[ij], Cij * (tu - sg), u[ij + 1] - u[ij - 1]);
     }
 }
 
